@@ -153,14 +153,16 @@ int qr_gemm_f32_add_norm(Context* c, float* y, const float* a, const float* x, i
  * `a` of rows x cols, 16-byte aligned). When cols % 32 == 0 the bridge keeps
  * the matrix's three-way BF16 split planes in MFMA fragment order (6 bytes per
  * element) and runs every qr_gemm / qr_gemm_f32_group / qr_gemm_f32_glu
- * projection of `a` over at least 64 tokens on its own BF16-MFMA kernel over
- * them (gemm_p3.hip: the six part products of the split, fp32 accumulation and
- * output, hence fp32 accuracy; a GLU of two prepared matrices with rows % 128
- * == 0 runs gate, up and the silu product as one kernel, gate_y and up_y
+ * projection of `a` over at least 5 tokens on its own BF16-MFMA kernels over
+ * them (gemm_kw.hip for up to a few hundred tokens, gemm_p3.hip beyond: the
+ * six part products of the split, fp32 accumulation and output, hence fp32
+ * accuracy; a GLU of two prepared matrices with rows % 128 == 0 (% 32 for few
+ * tokens) runs gate, up and the silu product as one kernel, gate_y and up_y
  * untouched). Other column counts prepare nothing (returns 0). The planes are
  * dropped by qr_gemm_f32_release(a), by qr_free(a), and by any qr_write /
- * qr_copy into the matrix's range; unprepared matrices take the split-BF16
- * kernel. */
+ * qr_copy into the matrix's range; unprepared matrices of up to a few
+ * hundred tokens take gemm_kw.hip too (split or widened as they load), others
+ * the split-BF16 kernel. */
 int qr_gemm_f32_prepare(Context* c, const float* a, int rows, int cols);
 int qr_gemm_f32_release(Context* c, const float* a);
 /* Prepared BF16 matrices (no counterpart in the reference's ABI; optional,
@@ -169,7 +171,7 @@ int qr_gemm_f32_release(Context* c, const float* a);
  * half of word i), 16-byte aligned. When cols % 32 == 0 the bridge keeps its
  * one plane in the same fragment order (2 bytes per element) and runs every
  * qr_gemm_bf16 / qr_gemm_bf16_group / qr_gemm_bf16_glu projection of it over
- * at least 64 tokens on the same kernels with three part products (x's three
+ * at least 5 tokens on the same kernels with three part products (x's three
  * planes times the exact BF16 weight). Released and invalidated as prepared
  * fp32 matrices (qr_gemm_f32_release takes either). */
 int qr_gemm_bf16_prepare(Context* c, const float* packed, int rows, int cols);
@@ -177,7 +179,7 @@ int qr_gemm_bf16_prepare(Context* c, const float* packed, int rows, int cols);
  * qr_gemm_bf16_prepare): `packed` is the reference's upload_int8 layout
  * (src/device.rs:550-561: rows fp32 scales, then the int8 values four per
  * word). The bridge keeps the values' one plane (integers are exact in BF16);
- * qr_gemm_i8 / qr_gemm_i8_group / qr_gemm_i8_glu over at least 64 tokens run
+ * qr_gemm_i8 / qr_gemm_i8_group / qr_gemm_i8_glu over at least 5 tokens run
  * the plane kernels and scale each output by its row's scale after the sum
  * (scale * sum(q x), as qr_gemm_i8). Released and invalidated as above. */
 int qr_gemm_i8_prepare(Context* c, const float* packed, int rows, int cols);

@@ -4,6 +4,7 @@
 // and the reference entry point each one replaces: include/qwen_bridge.h.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -73,6 +74,9 @@ struct Context {
     const float* xp_src = nullptr;
     int xp_rows = 0, xp_cols = 0;
     unsigned long serial = 0, xp_serial = 0;
+    // Widths of inputs that a projection split itself (split_input), the
+    // first 16 of them.
+    int plane_widths[16] = {}, plane_width_count = 0;
     // The width of the projection that took the last RmsNormGate output right
     // after it (its rows span several groups), by group size: from then on such
     // a norm writes its planes in rows of that width.
@@ -190,19 +194,39 @@ int ensure(Context* c, float** buf, size_t* len, size_t need, const char* what) 
 const void* i8_packed(const float* packed) { return packed; }
 
 // ---- prepared fp32 and BF16 matrices (csrc/gemm_p3.hip)
-// Projections of at least this many tokens take the P3 planes when their
-// matrix is prepared (fewer tokens: the split-BF16 kernel, whose tiles the
-// small batches fill as well).
-constexpr int kPlanesMinBatch = 64;
+// Projections of at least this many tokens (fewer: the GEMV kernels) take
+// their input as planes when their matrix is prepared, or its format allows.
+constexpr int kPlanesMinBatch = 5;
+// Prepared matrices outside kw_wanted's range take the prefill GEMM from this
+// many tokens on.
+constexpr int kPrefillMinBatch = 64;
 
 // The prepared planes of matrix a of format t (fp32: three planes; BF16 and
 // int8: one).
-const Context::Prepared* prepared_for(Context* c, qr::WeightType t, const void* a, int rows, int cols, int batch) {
-    if (batch < kPlanesMinBatch || rows <= 16) return nullptr;
+const Context::Prepared* planes_of(Context* c, qr::WeightType t, const void* a, int rows, int cols) {
+    if (rows <= 16) return nullptr;
     auto it = c->prepared.find(static_cast<const float*>(a));
     if (it == c->prepared.end() || it->second.rows != rows || it->second.cols != cols || it->second.kind != t)
         return nullptr;
     return &it->second;
+}
+const Context::Prepared* prepared_for(Context* c, qr::WeightType t, const void* a, int rows, int cols, int batch) {
+    return batch < kPrefillMinBatch ? nullptr : planes_of(c, t, a, rows, cols);
+}
+// Matrix a as an operand of the few-token kernels (gemm_kw.hip): its planes,
+// or the matrix itself; false when they do not take it.
+bool kw_item(Context* c, qr::WeightType t, float* y, const void* a, const float* x, int rows, int cols, int batch,
+             qr::KwItem* out) {
+    if (batch < kPlanesMinBatch || !qr::p3_cols_ok(cols) || reinterpret_cast<uintptr_t>(x) % 16 != 0) return false;
+    const float* scale = t == qr::WeightType::I8 ? static_cast<const float*>(a) : nullptr;
+    if (const Context::Prepared* p = planes_of(c, t, a, rows, cols)) {
+        *out = qr::KwItem{y, p->w3, p->scales, rows, false};
+    } else if (qr::kw_raw_ok(t, a, rows, cols)) {
+        *out = qr::KwItem{y, scale ? static_cast<const void*>(scale + rows) : a, scale, rows, true};
+    } else {
+        return false;
+    }
+    return qr::kw_wanted(t, out->raw, batch, rows);
 }
 // A planes buffer large enough for batch rows of cols (queued work on the old
 // buffer drains first).
@@ -224,6 +248,10 @@ int grow_xp(Context* c, int cols, int batch) {
     if (qr::p3_elements(batch, cols) > c->xp_len) c->xp_src = nullptr;
     return grow_planes(c, &c->xp, &c->xp_len, cols, batch);
 }
+bool split_width(const Context* c, int cols) {
+    const int* end = c->plane_widths + c->plane_width_count;
+    return std::find(c->plane_widths, end, cols) != end;
+}
 // x's P3 planes into c->xp: already there when the previous bridge call
 // produced x with them, else split now.
 int split_input(Context* c, const float* x, int cols, int batch) {
@@ -231,14 +259,19 @@ int split_input(Context* c, const float* x, int cols, int batch) {
         c->gate_width[c->gate_d] = cols;  // a gated norm's output projected: its row width
     if (c->xp_src == x && c->xp_rows == batch && c->xp_cols == cols && c->xp_serial + 1 == c->serial) return 0;
     c->xp_src = nullptr;
+    if (!split_width(c, cols) && c->plane_width_count < 16)  // from now on this width's producers write the planes
+        c->plane_widths[c->plane_width_count++] = cols;
     if (int st = grow_xp(c, cols, batch)) return st;
     auto s = scope(c, [&] { return std::string("p3_split ") + shape(batch, cols, 1); });
     return launched(c, "p3_split", qr::p3_split(c->stream, c->xp, x, batch, cols));
 }
 // Whether a producer of `rows` rows of width `cols` should also write the
-// planes: enough rows for the planes path and a prepared matrix of that width.
+// planes: enough rows for the planes path, and a prepared matrix of that width
+// or (while the few-token kernels take matrices without planes) a projection
+// that split such an input before.
 bool planes_wanted(Context* c, int cols, int rows) {
     if (rows < kPlanesMinBatch || !qr::p3_cols_ok(cols)) return false;
+    if (rows <= qr::kKwMaxTokens && split_width(c, cols)) return true;
     for (auto& kv : c->prepared)
         if (kv.second.cols == cols && kv.second.rows > 16) return true;
     return false;
@@ -311,6 +344,12 @@ int rope_table(Context* c, float theta, int rot, const float** out) {
 
 int project(Context* c, qr::WeightType t, float* y, const void* a, const float* x, int rows, int cols, int batch) {
     if (rows < 1 || cols < 1 || batch < 1) return fail(c, "projection shape", -1);
+    qr::KwItem kw;
+    if (kw_item(c, t, y, a, x, rows, cols, batch, &kw)) {
+        if (int st = split_input(c, x, cols, batch)) return st;
+        auto s = scope(c, [&] { return std::string("gemm_") + wname(t) + "_kw " + shape(rows, cols, batch); });
+        return launched(c, "gemm_kw", qr::kw_gemm(c->stream, t, &kw, 1, c->xp, batch, cols));
+    }
     if (const Context::Prepared* p = prepared_for(c, t, a, rows, cols, batch)) {
         if (int st = split_input(c, x, cols, batch)) return st;
         return p3_project(c, y, *p, batch);
@@ -332,8 +371,26 @@ int group(Context* c, qr::WeightType t, int n, const QrProjection* items, const 
     for (int i = 0; i < n; ++i)
         if (items[i].rows < 1) return fail(c, "GEMM group shape", -1);
     if (qr::gemm_preferred(t, items[0].rows, cols, batch)) {
-        bool split = false;  // x's planes, made at the group's first prepared matrix
+        bool split = false;  // x's planes, made at the group's first matrix that takes them
+        // the matrices of the few-token kernels, up to kKwItems to a launch
+        qr::KwItem kw[qr::kKwItems], it;
+        auto few = [&](int i) { return kw_item(c, t, items[i].y, items[i].a, x, items[i].rows, cols, batch, &it); };
+        for (int i = 0, m = 0; i < n; ++i) {
+            if (few(i)) kw[m++] = it;
+            if (m == 0 || (m < qr::kKwItems && i + 1 < n)) continue;
+            if (!split)
+                if (int st = split_input(c, x, cols, batch)) return st;
+            split = true;
+            auto s = scope(c, [&] {
+                std::string l = std::string("gemm_") + wname(t) + "_kw_group";
+                for (int k = 0; k < m; ++k) l += (k ? "+" : " ") + shape(kw[k].rows, cols, 1);
+                return l + " t" + std::to_string(batch);
+            });
+            if (int st = launched(c, "gemm_kw", qr::kw_gemm(c->stream, t, kw, m, c->xp, batch, cols))) return st;
+            m = 0;
+        }
         for (int i = 0; i < n; ++i) {
+            if (few(i)) continue;
             if (const Context::Prepared* p = prepared_for(c, t, items[i].a, items[i].rows, cols, batch)) {
                 if (!split) {
                     if (int st = split_input(c, x, cols, batch)) return st;
@@ -343,7 +400,7 @@ int group(Context* c, qr::WeightType t, int n, const QrProjection* items, const 
                 continue;
             }
             // two consecutive few-row fp32 or BF16 matrices (the DeltaNet a / b) in one launch
-            if (i + 1 < n && qr::gemm_ab_ok(t, items[i].a, x, items[i].rows, cols, batch) &&
+            if (i + 1 < n && !few(i + 1) && qr::gemm_ab_ok(t, items[i].a, x, items[i].rows, cols, batch) &&
                 qr::gemm_ab_ok(t, items[i + 1].a, x, items[i + 1].rows, cols, batch)) {
                 auto sc = scope(c, [&] {
                     return std::string("gemm_") + wname(t) + "_ab " + shape(items[i].rows, cols, batch) + "+" +
@@ -379,6 +436,27 @@ int glu(Context* c, qr::WeightType t, float* product, float* gate_y, float* up_y
     if (!qr::gemm_preferred(t, rows, cols, batch)) {
         auto s = scope(c, [&] { return std::string("gemv_") + wname(t) + "_glu 2x" + shape(rows, cols, batch); });
         return launched(c, "gemv_glu", qr::gemv_glu(c->stream, t, product, gate, up, x, rows, cols, batch));
+    }
+    {
+        // a few to a few hundred tokens: one kernel over the matrices' planes or the matrices themselves
+        qr::KwItem kg, ku;
+        if (rows % 32 == 0 && reinterpret_cast<uintptr_t>(product) % 16 == 0 &&
+            kw_item(c, t, product, gate, x, rows, cols, batch, &kg) &&
+            kw_item(c, t, product, up, x, rows, cols, batch, &ku) && kg.raw == ku.raw &&
+            qr::kw_wanted(t, kg.raw, batch, 2 * rows)) {
+            if (int st = split_input(c, x, cols, batch)) return st;
+            const bool planes = planes_wanted(c, rows, batch);
+            if (planes)
+                if (int st = grow_planes(c, &c->xp_alt, &c->xp_alt_len, rows, batch)) return st;
+            auto s = scope(c, [&] { return std::string("gemm_") + wname(t) + "_kw_glu 2x" + shape(rows, cols, batch); });
+            const int st = qr::kw_glu(c->stream, t, product, planes ? c->xp_alt : nullptr, kg, ku, c->xp, batch, cols);
+            if (st == 0 && planes) {
+                std::swap(c->xp, c->xp_alt);
+                std::swap(c->xp_len, c->xp_alt_len);
+                planes_made(c, product, batch, rows);
+            }
+            return launched(c, "gemm_kw_glu", st);
+        }
     }
     {
         const Context::Prepared* pg = prepared_for(c, t, gate, rows, cols, batch);

@@ -128,6 +128,31 @@ int p3_gemm_glu(hipStream_t s, float* product, __bf16* planes, const __bf16* xp,
                 const float* scale_up = nullptr);
 size_t p3_glu_scratch(int M, int rows, int K, int wplanes = 3);
 
+// gemm_kw.hip -----------------------------------------------------------------
+// The projections of a few to a few hundred tokens: K split over the waves of
+// a block. X as its P3 planes; each matrix as its planes (3 for fp32, 1 for
+// BF16 / int8) or in its own format (raw: fp32, packed BF16, or the int8
+// values that follow the scales; kw_raw_ok), K % 32 == 0. int8: `scale` the
+// row scales, applied after the sum.
+constexpr int kKwItems = 8, kKwMaxTokens = 640;
+struct KwItem {
+    float* y;
+    const void* w;
+    const float* scale;
+    int rows;
+    bool raw;
+};
+// Whether a projection of M tokens and so many rows (the GLU: gate's and up's
+// together) runs faster here than on the prefill GEMMs.
+bool kw_wanted(WeightType t, bool raw, int M, int rows);
+// Whether a matrix without planes has the alignment the kernels load it by.
+bool kw_raw_ok(WeightType t, const void* a, int rows, int cols);
+int kw_gemm(hipStream_t s, WeightType t, const KwItem* items, int n, const __bf16* xp, int M, int K);
+// product = silu(X G^T) * (X U^T) and, when set, its P3 planes; rows % 32 == 0,
+// product 16-byte aligned.
+int kw_glu(hipStream_t s, WeightType t, float* product, __bf16* planes, const KwItem& gate, const KwItem& up,
+           const __bf16* xp, int M, int K);
+
 // Y1 = X A1^T and (rows2 > 0) Y2 = X A2^T in one launch for fp32 (or packed
 // BF16 / int8, cols % 16 == 0) matrices of at most 16 rows and 1024 columns
 // (the DeltaNet a / b projections of prefill), when gemm_ab_ok holds for each.

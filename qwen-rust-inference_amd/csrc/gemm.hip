@@ -1,5 +1,7 @@
 // Prefill projections Y[batch, rows] = X[batch, cols] . A^T (batch >= 5) on
-// gfx950, fp32 / BF16 / int8-per-row weights, fp32 accumulation.
+// gfx950, fp32 / BF16 / int8-per-row weights, fp32 accumulation: what neither
+// the few-token kernels (gemm_kw.hip: cols % 32 == 0, up to 640 tokens) nor
+// the planes GEMM (gemm_p3.hip: prepared matrices) take.
 //
 // fp32 weights (the prefill of every config): BF16 MFMA
 // (v_mfma_f32_32x32x16_bf16) on operands split into three BF16 parts each,
