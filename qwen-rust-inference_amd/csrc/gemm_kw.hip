@@ -11,9 +11,9 @@
 // projection of 128 tokens has 8 such tiles), and cutting K into chunks over
 // blocks costs partials in memory and a second launch. Here a block owns a
 // small output tile over the whole K: wave w takes the 16-deep k tiles w, w +
-// 8, ..., its operands straight from L2 / HBM into registers (a fragment is
+// 4, ..., its operands straight from L2 / HBM into registers (a fragment is
 // one 16-byte load per lane, 1 KiB contiguous per wave; the next k tile's in
-// flight while one is multiplied), and the eight partial tiles are added in
+// flight while one is multiplied), and the four partial tiles are added in
 // wave order through LDS: no staging, no barrier in the loop, one launch,
 // results independent of timing.
 //
@@ -27,11 +27,11 @@
 // Measured (one call, weights cold, launch included; before: the prefill GEMM
 // of gemm_p3.hip over planes, or gemm_bf3_kernel under 64 tokens and for
 // matrices without planes):
-//   GLU 2 x 3584 x 1024, fp32 planes: 23 tokens 70.4 -> 13.4 us, 128 tokens 28 -> 18
-//   GLU, BF16 plane: 23 tokens 54.6 -> 7.7 us, 128 tokens 24 -> 11.7
-//   GLU, int8 without a plane, 128 tokens: 59 -> 12.6 us
-//   down 1024 x 3584, fp32 planes: 23 tokens 24.6 -> 12.2 us, 128 tokens 22.4 -> 13.0
-//   q|k|v|z 8192 x 1024, fp32 planes, 128 tokens: 26 -> 18 us; BF16 21.5 -> 10.2
+//   GLU 2 x 3584 x 1024, fp32 planes: 23 tokens 70.2 -> 14.2 us, 128 tokens 25.1 -> 17.3
+//   GLU, BF16 plane: 23 tokens 54.1 -> 7.2 us, 128 tokens 25.1 -> 11.2, 512 tokens 38.3 -> 29.6
+//   GLU, int8 without a plane, 128 tokens: 59.5 -> 12.6 us
+//   down 1024 x 3584, fp32 planes: 23 tokens 24.8 -> 12.1 us, 128 tokens 22.2 -> 12.9
+//   q|k|v 5120 x 1024, 128 tokens: fp32 planes 17.2 -> 12.3 us, BF16 19.4 -> 9.6
 #include <type_traits>
 
 #include "common.h"
@@ -43,7 +43,11 @@ typedef float f16v __attribute__((ext_vector_type(16)));
 typedef float f4v __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-constexpr int NW = 8;  // waves per block
+// Waves per block. Two blocks of four share a CU (their registers and LDS allow
+// it), so a launch of a few more tiles than CUs runs on: against one block of
+// eight waves, 130 column tiles at 128 tokens 28.1 -> 23.8 us (fp32) and 16.5 ->
+// 13.4 (BF16), the BF16 GLU of 512 tokens 34.9 -> 29.6, one round the same.
+constexpr int NW = 4;
 
 // One launch: up to kKwItems matrices of one X (their column tiles in order).
 struct KwArgs {
@@ -133,8 +137,8 @@ __device__ __forceinline__ void products(F&& mfma) {
     }
 }
 
-// n steps through a ring of NS register buffers: load(buffer, step) NS steps
-// ahead of multiply(buffer). The main loop's loads are unconditional (a join
+// n steps through a ring of NS (even) register buffers: load(buffer, step) NS
+// steps ahead of multiply(buffer, step % 2). The main loop's loads are unconditional (a join
 // between a path with loads and one without would make the compiler wait for
 // more than the buffer it needs).
 template <int NS, class Buf, class L, class M>
@@ -146,29 +150,32 @@ __device__ __forceinline__ void ring(int n, L&& load, M&& multiply) {
     for (; s + 2 * NS <= n; s += NS)
 #pragma unroll
         for (int i = 0; i < NS; ++i) {
-            multiply(b[i]);
+            multiply(b[i], i % 2);
             load(b[i], s + i + NS);
         }
 #pragma unroll
     for (int i = 0; i < NS; ++i)
         if (s + i < n) {
-            multiply(b[i]);
+            multiply(b[i], i % 2);
             if (s + i + NS < n) load(b[i], s + i + NS);
         }
     s += NS;
 #pragma unroll
     for (int i = 0; i < NS - 1; ++i)
-        if (s + i < n) multiply(b[i]);
+        if (s + i < n) multiply(b[i], i % 2);
 }
 
-// Wave w's k tiles (w, w + 8, ...) of a (32 TMT) x (32 TNT) tile into acc. xb
-// / wb: this lane's address of each 32-row tile's k tile 0.
+// Wave w's k tiles (w, w + NW, ...) of a (32 TMT) x (32 TNT) tile into acc. xb
+// / wb: this lane's address of each 32-row tile's k tile 0. Even and odd steps
+// sum in accumulators of their own: the chain of fp32 additions behind a sum is
+// K / 128 k tiles long, as with eight waves (error against 64 bits, DeltaNet
+// layer of 128 fp32 tokens: 6.6e-7 with one chain).
 template <WeightType T, bool RAW, int TMT, int TNT>
 __device__ __forceinline__ void k_wave(f16v (&acc)[TMT][TNT], const char* const (&xb)[TMT], const char* const (&wb)[TNT],
                                        int kt, int w) {
     constexpr int XSTEP = 3 * 1024, WSTEP = RAW ? 16 * kRawBytes<T> : kPlanes<T> * 1024;
     const int n = (kt - w + NW - 1) / NW;
-    constexpr int NS = TMT * TNT == 4 ? 2 : TMT * TNT == 2 ? 3 : 4;  // buffers that fit 256 VGPRs
+    constexpr int NS = TMT * TNT == 4 ? 2 : 4;  // buffers that fit 256 VGPRs
     struct Buf {
         bf16x8 x[TMT][3];
         WReg<T, RAW> w[TNT];
@@ -182,7 +189,14 @@ __device__ __forceinline__ void k_wave(f16v (&acc)[TMT][TNT], const char* const 
 #pragma unroll
             for (int q = 0; q < 3; ++q) b.x[i][q] = *reinterpret_cast<const bf16x8*>(xb[i] + k * XSTEP + 1024 * q);
     };
-    auto multiply = [&](const Buf& b) {
+    f16v odd[TMT][TNT];
+#pragma unroll
+    for (int i = 0; i < TMT; ++i)
+#pragma unroll
+        for (int j = 0; j < TNT; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = odd[i][j][r] = 0.f;
+    auto multiply = [&](const Buf& b, int parity) {
         bf16x8 h[TNT][kPlanes<T>];
 #pragma unroll
         for (int j = 0; j < TNT; ++j) wplanes<T, RAW>(b.w[j], h[j]);
@@ -190,11 +204,17 @@ __device__ __forceinline__ void k_wave(f16v (&acc)[TMT][TNT], const char* const 
 #pragma unroll
             for (int i = 0; i < TMT; ++i)
 #pragma unroll
-                for (int j = 0; j < TNT; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.x[i][px], h[j][pw], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < TNT; ++j) {
+                    f16v& a = parity ? odd[i][j] : acc[i][j];
+                    a = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.x[i][px], h[j][pw], a, 0, 0, 0);
+                }
         });
     };
     if (w < kt) ring<NS, Buf>(n, load, multiply);
+#pragma unroll
+    for (int i = 0; i < TMT; ++i)
+#pragma unroll
+        for (int j = 0; j < TNT; ++j) acc[i][j] += odd[i][j];
 }
 
 // Block b's tile: the 8 XCDs take blocks in turn; XCD x takes column tiles x,
@@ -234,10 +254,14 @@ __device__ __forceinline__ void store4(const KwArgs::Item& it, int m, int n, f4v
     }
 }
 
+// Two waves per SIMD (256 registers each) also keep the accumulators out of the
+// AGPRs: with 512 registers to a wave the compiler moved them there and back at
+// every branch of the ring's end and read the last one before its MFMA had
+// written it.
 // GLU = false: a (32 TMT) x (32 TNT) tile of one item. GLU = true (TNT = 2):
 // 32 gate rows and the same 32 up rows, product = silu(g) * u and its planes.
 template <WeightType T, int TMT, int TNT, bool GLU>
-__global__ __launch_bounds__(64 * NW) void kw_kernel(KwArgs p) {
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) void kw_kernel(KwArgs p) {
     constexpr int TM = 32 * TMT, TN = 32 * TNT, PITCH = TN + 4, SLOT = TM * PITCH;
     __shared__ __attribute__((aligned(16))) float part[NW * SLOT];
     int mt, nt;
@@ -252,14 +276,15 @@ __global__ __launch_bounds__(64 * NW) void kw_kernel(KwArgs p) {
     for (int i = 0; i < TMT; ++i)
         xb[i] = reinterpret_cast<const char*>(p.xp) + size_t(mt * TMT + i) * kt * 3072 + 16 * lane;
     f16v acc[TMT][TNT];
-#pragma unroll
-    for (int i = 0; i < TMT; ++i)
-#pragma unroll
-        for (int j = 0; j < TNT; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
     const char* wb[TNT];
-    if (it.raw) {
+    if (!GLU && TNT == 2 && it.raw && it.rows <= 32) {  // a few-row matrix (the DeltaNet a and b): half the tile
+        const char* wb1[1] = {reinterpret_cast<const char*>(it.w) +
+                              (size_t(min(lane & 31, it.rows - 1)) * kt * 16 + 8 * (lane >> 5)) * kRawBytes<T>};
+        f16v half[TMT][1];
+        k_wave<T, true, TMT, 1>(half, xb, wb1, kt, w);
+#pragma unroll
+        for (int i = 0; i < TMT; ++i) acc[i][0] = acc[i][TNT - 1] = half[i][0];  // (columns past the matrix: not stored)
+    } else if (it.raw) {
 #pragma unroll
         for (int j = 0; j < TNT; ++j) {  // rows past the matrix read its last row (not stored)
             const int row = min(n0 + (GLU ? 0 : 32 * j) + (lane & 31), it.rows - 1);
@@ -337,11 +362,11 @@ __global__ __launch_bounds__(64 * NW) void kw_narrow_kernel(KwArgs p) {
     // fragment lane of row r16 (of 16) and this lane's k: r16 + 32 ((l / 16) % 2), k tile l / 32 of the step
     const int fl = (lane & 15) + 32 * ((lane >> 4) & 1), fk = lane >> 5;
     const char* xb = reinterpret_cast<const char*>(p.xp) + (size_t(mt) * kt + fk) * 3072 + 16 * fl;
-    f4v acc[2];
+    f4v acc[2][2];  // [row half][even, odd steps]
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc[i][r] = 0.f;
+        for (int r = 0; r < 4; ++r) acc[i][0][r] = acc[i][1][r] = 0.f;
     auto run = [&](auto raw, const char* wb) {
         constexpr bool RAW = decltype(raw)::value;
         constexpr int WSTEP = RAW ? 32 * kRawBytes<T> : 2 * WP * 1024;
@@ -358,16 +383,17 @@ __global__ __launch_bounds__(64 * NW) void kw_narrow_kernel(KwArgs p) {
                 for (int q = 0; q < 3; ++q)
                     b.x[i][q] = *reinterpret_cast<const bf16x8*>(xb + s * 6144 + 1024 * q + 256 * i);
         };
-        auto multiply = [&](const Buf& b) {
+        auto multiply = [&](const Buf& b, int parity) {
             bf16x8 h[WP];
             wplanes<T, RAW>(b.w, h);
             products<T>([&](int px, int pw) {
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
-                    acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b.x[i][px], h[pw], acc[i], 0, 0, 0);
+                    acc[i][parity] =
+                        __builtin_amdgcn_mfma_f32_16x16x32_bf16(b.x[i][px], h[pw], acc[i][parity], 0, 0, 0);
             });
         };
-        if (w < steps) ring<3, Buf>((steps - w + NW - 1) / NW, load, multiply);
+        if (w < steps) ring<4, Buf>((steps - w + NW - 1) / NW, load, multiply);
     };
     if (it.raw) {
         const int row = min(n0 + (lane & 15), it.rows - 1);
@@ -380,7 +406,7 @@ __global__ __launch_bounds__(64 * NW) void kw_narrow_kernel(KwArgs p) {
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-            part[w * SLOT + (16 * i + 4 * (lane >> 4) + r) * PITCH + (lane & 15)] = acc[i][r];
+            part[w * SLOT + (16 * i + 4 * (lane >> 4) + r) * PITCH + (lane & 15)] = acc[i][0][r] + acc[i][1][r];
     __syncthreads();
     if (tid < TM * TN / 4) {
         const int m = tid / (TN / 4), c = tid % (TN / 4) * 4;
@@ -445,14 +471,15 @@ Tile pick_tile(WeightType t, const KwItem* items, int n, int M) {
 
 }  // namespace
 
-// Up to kKwMaxTokens tokens, and while the 64 x 64 tiles number at most 512
-// (three planes: 640 of them take as long as the prefill GEMM's 128 x 256
-// tiles, 42.6 and 45.6 us at 300 tokens of 8192 rows; 1024 of them 62 against
-// 49) or 1024 (one plane, or no planes at all: 896 of the GLU at 512 tokens
-// 34.5 against 38.7 us; 1792 of them 82 against 57).
+// Up to kKwMaxTokens tokens, and while the 64 x 64 tiles number at most 640
+// (three planes; against the prefill GEMM's 128 x 256 tiles: 560 of the GLU at
+// 300 tokens 38.8 against 42.3 us, 640 of q|k|v at 512 tokens 35.9 against
+// 40.2, 1024 of 8192 rows at 512 tokens 62 against 49) or 1152 (one plane, or
+// no planes at all: 896 of the GLU at 512 tokens 29.6 against 38.3 us; 1792 of
+// them at 1024 tokens 82 against 57).
 bool kw_wanted(WeightType t, bool raw, int M, int rows) {
     const long tiles = long(ceil_div(M, 64)) * long(ceil_div(rows, 64));
-    return M <= kKwMaxTokens && (M <= 64 || tiles <= (t == WeightType::F32 && !raw ? 512 : 1024));
+    return M <= kKwMaxTokens && (M <= 64 || tiles <= (t == WeightType::F32 && !raw ? 640 : 1152));
 }
 
 bool kw_raw_ok(WeightType t, const void* a, int rows, int cols) {
@@ -484,7 +511,7 @@ int kw_glu(hipStream_t s, WeightType t, float* product, __bf16* planes, const Kw
         (reinterpret_cast<uintptr_t>(product) | reinterpret_cast<uintptr_t>(gate.scale) |
          reinterpret_cast<uintptr_t>(up.scale)) % 16)
         return int(hipErrorInvalidValue);
-    // one plane: 32-token tiles also past one round of 64-token ones (300 tokens 25.4 against 28.9 us)
+    // one plane: 32-token tiles also past one round of 64-token ones (300 tokens 25 against 29 us)
     const long cols = gate.rows / 32, small = cols * ceil_div(M, 32), large = cols * ceil_div(M, 64);
     const Tile tile = small <= 256 || (large > 256 && t != WeightType::F32 && !gate.raw) ? k32x64 : k64x64;
     KwArgs a{};
