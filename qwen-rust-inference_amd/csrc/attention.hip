@@ -30,9 +30,10 @@ struct ReadArgs {
     int d, heads, kv, length0, rows, span, splits, tiles;
 };
 
+// Head dims under 64 (larger ones: attention_decode_kernel).
 template <int D, int G>
 __global__ __launch_bounds__(256) void attention_read_kernel(ReadArgs a) {
-    constexpr int DPL = D >= 64 ? 16 : 4;  // floats per lane
+    constexpr int DPL = 4;                  // floats per lane
     constexpr int LPP = D / DPL;            // lanes per position
     constexpr int PPW = 64 / LPP;           // positions per wave per step
     const int split = blockIdx.x, kvh = blockIdx.y, row = blockIdx.z;
@@ -155,77 +156,242 @@ __global__ __launch_bounds__(256) void attention_read_kernel(ReadArgs a) {
     }
 }
 
-// Merge the split partials: LANES lanes (1, or the 4 of a quad) per (row,
-// head, 4 dims), lane q taking splits q, q + LANES, ... and a quad's (max,
-// sum, weighted sums) combined by two xor shuffles. Quads for a decode row
-// (tens of splits: each lane's loads in flight together), one lane for a
-// prefill chunk (a few shares: more lanes only add shuffles). The partial
-// sums are read as 8-byte pairs (a partial is d + 2 floats: even, not a
-// multiple of 4). The order of every sum is fixed for a given split count.
-template <int LANES>
-__global__ __launch_bounds__(256) void attention_combine_kernel(ReadArgs a) {
-    typedef float f2v __attribute__((ext_vector_type(2)));
+// The same decomposition for head dims of 64 and more (a decode row of the
+// models), with nothing of a context vector crossing lanes until the end. A
+// chunk of CH positions at a time: each wave scores its CPW positions (LPP
+// lanes to a position, 16 dims each), one wave per query head turns the
+// chunk's scores into probabilities against the running maximum, and each wave
+// adds its own positions' values, lane l holding dims 4 (l % VL) .. + 3 of
+// position l / VL. K and V of the next chunk are loaded before the current one
+// is scored and weighted. The waves' sums meet in LDS once per block.
+// Bounded by its chain of loads, barriers and exponentials, not by bytes: at
+// 8192 positions (16.8 MB of K/V) 10.8 us, against 16.2 for the kernel above,
+// whose position slots merge every context value through lane shuffles.
+template <int D, int G>
+__global__ __launch_bounds__(256) void attention_decode_kernel(ReadArgs a) {
     typedef float f4v __attribute__((ext_vector_type(4)));
-    static_assert(LANES == 1 || LANES == 4 || LANES == 16, "one lane, a quad or 16 lanes");
-    const long idx = blockIdx.x * long(blockDim.x) + threadIdx.x;
-    const int q = a.d / 4;
-    const long total = long(a.rows) * a.heads * q * LANES;  // whole quads: the shuffles see only live lanes
-    if (idx >= total) return;
-    const int lq = int(idx % LANES);
-    const long e = idx / LANES;
-    const int i = 4 * int(e % q);
-    const long rh = e / q;  // row * heads + head
-    const float* parts = a.parts + size_t(rh) * a.splits * (a.d + 2);
-    float mm = -INFINITY;
-#pragma unroll 8
-    for (int s = lq; s < a.splits; s += LANES) mm = fmaxf(mm, parts[size_t(s) * (a.d + 2)]);
+    constexpr int LPP = D / 16, PPW = 64 / LPP;        // lanes per position, positions per wave and score step
+    constexpr int CPW = PPW > 8 ? PPW : 8, KS = CPW / PPW;  // positions per wave and chunk, score steps
+    constexpr int CH = 4 * CPW, VL = D / 4, VP = 64 / VL, VS = CPW / VP;
+    __shared__ float ss[2][CH][G], corr[2][G];
+    __shared__ float sm[G], sl[G];
+    __shared__ f4v sacc[4][G][VL];
+    const int split = blockIdx.x, kvh = blockIdx.y, row = blockIdx.z;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int sub = lane % LPP, slot = lane / LPP, vl = lane % VL, vslot = lane / VL;
+    const int length = a.length0 + row;
+    const int begin = split * a.span, end = min(length, begin + a.span);
+    const float scale = 1.f / sqrtf(float(D));
+    const size_t rowstride = size_t(a.kv) * D;
+    const float* kbase = a.keys + size_t(kvh) * D + 4 * sub;
+    const float* vbase = a.values + size_t(kvh) * D + 4 * vl;
+    f4v kx[KS][4], vx[VS];
+    // a position past the span reads its first row (and is not used)
+    auto load_k = [&](int c0) {
 #pragma unroll
-    for (int o = 1; o < LANES; o <<= 1) mm = fmaxf(mm, __shfl_xor(mm, o, 64));
-    float den = 0.f;
-    f4v num = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-    for (int s = lq; s < a.splits; s += LANES) {
-        const float* p = parts + size_t(s) * (a.d + 2);
-        const float c = p[0] == -INFINITY ? 0.f : expf(p[0] - mm);
-        den += p[1] * c;
-        const f2v lo = *reinterpret_cast<const f2v*>(p + 2 + i), hi = *reinterpret_cast<const f2v*>(p + 4 + i);
-        num.x += lo.x * c;
-        num.y += lo.y * c;
-        num.z += hi.x * c;
-        num.w += hi.y * c;
-    }
-    if constexpr (LANES > 1) {
+        for (int s = 0; s < KS; ++s) {
+            const int p = c0 + CPW * wave + PPW * s + slot;
+            const float* kp = kbase + size_t(p < end ? p : begin) * rowstride;
 #pragma unroll
-        for (int o = 1; o < LANES; o <<= 1) {
-            den += __shfl_xor(den, o, 64);
-            num.x += __shfl_xor(num.x, o, 64);
-            num.y += __shfl_xor(num.y, o, 64);
-            num.z += __shfl_xor(num.z, o, 64);
-            num.w += __shfl_xor(num.w, o, 64);
+            for (int e = 0; e < 4; ++e) kx[s][e] = *reinterpret_cast<const f4v*>(kp + 4 * LPP * e);
         }
-        if (lq != 0) return;
+    };
+    auto load_v = [&](int c0) {
+#pragma unroll
+        for (int s = 0; s < VS; ++s) {
+            const int p = c0 + CPW * wave + VP * s + vslot;
+            vx[s] = *reinterpret_cast<const f4v*>(vbase + size_t(p < end ? p : begin) * rowstride);
+        }
+    };
+    load_k(begin);
+    f4v q[G][4];  // dims 4 sub + 4 LPP e .. + 3
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            q[g][e] = *reinterpret_cast<const f4v*>(a.query + (size_t(row) * a.heads + size_t(kvh) * G + g) * D +
+                                                    4 * sub + 4 * LPP * e);
+    load_v(begin);
+    f4v acc[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) acc[g] = f4v{0.f, 0.f, 0.f, 0.f};
+    constexpr int HW = (G + 3) / 4;  // heads whose softmax this wave keeps: wave, wave + 4, ...
+    float m[HW], l[HW];
+#pragma unroll
+    for (int i = 0; i < HW; ++i) {
+        m[i] = -INFINITY;
+        l[i] = 0.f;
     }
-    const size_t o = size_t(rh) * a.d + i;
-    const f4v g = *reinterpret_cast<const f4v*>(a.gate + o);
-    f4v r;
-    r.x = (num.x / den) * sigmoidf_(g.x);
-    r.y = (num.y / den) * sigmoidf_(g.y);
-    r.z = (num.z / den) * sigmoidf_(g.z);
-    r.w = (num.w / den) * sigmoidf_(g.w);
-    *reinterpret_cast<f4v*>(a.out + o) = r;
+    int b = 0;
+    for (int c0 = begin; c0 < end; c0 += CH, b ^= 1) {
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            const int i = CPW * wave + PPW * s + slot;
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                float t = 0.f;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) t = fmaf(q[g][e][d], kx[s][e][d], t);
+                t = group_sum<LPP>(t) * scale;
+                if (sub == 0) ss[b][i][g] = c0 + i < end ? t : -INFINITY;
+            }
+        }
+        if (c0 + CH < end) load_k(c0 + CH);
+        __syncthreads();
+#pragma unroll
+        for (int h = 0; h < HW; ++h) {
+            const int g = wave + 4 * h;
+            if (g >= G) break;
+            const float x = lane < CH ? ss[b][lane][g] : -INFINITY;
+            const float mn = fmaxf(m[h], wave_max(x));  // finite: the chunk's first position is live
+            const float c = expf(m[h] - mn), w = expf(x - mn);
+            l[h] = l[h] * c + wave_sum(w);
+            m[h] = mn;
+            if (lane < CH) ss[b][lane][g] = w;
+            if (lane == 0) corr[b][g] = c;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int g = 0; g < G; ++g) acc[g] *= corr[b][g];
+#pragma unroll
+        for (int s = 0; s < VS; ++s) {
+            const int i = CPW * wave + VP * s + vslot;
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const float w = ss[b][i][g];
+#pragma unroll
+                for (int d = 0; d < 4; ++d) acc[g][d] = fmaf(w, vx[s][d], acc[g][d]);
+            }
+        }
+        if (c0 + CH < end) load_v(c0 + CH);
+    }
+#pragma unroll
+    for (int o = VL; o < 64; o <<= 1)
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int d = 0; d < 4; ++d) acc[g][d] += __shfl_xor(acc[g][d], o, 64);
+    if (vslot == 0)
+#pragma unroll
+        for (int g = 0; g < G; ++g) sacc[wave][g][vl] = acc[g];
+#pragma unroll
+    for (int h = 0; h < HW; ++h)
+        if (wave + 4 * h < G && lane == 0) {
+            sm[wave + 4 * h] = m[h];
+            sl[wave + 4 * h] = l[h];
+        }
+    __syncthreads();
+    for (int o = int(threadIdx.x); o < G * VL; o += 256) {
+        const int g = o / VL, i = 4 * (o % VL), head = kvh * G + g;
+        const f4v num = (sacc[0][g][o % VL] + sacc[1][g][o % VL]) + (sacc[2][g][o % VL] + sacc[3][g][o % VL]);
+        if (a.splits == 1) {
+            const size_t at = (size_t(row) * a.heads + head) * D + i;
+#pragma unroll
+            for (int d = 0; d < 4; ++d) a.out[at + d] = (num[d] / sl[g]) * sigmoidf_(a.gate[at + d]);
+        } else {
+            float* part = a.parts + ((size_t(row) * a.heads + head) * a.splits + split) * (D + 2);
+            if (i == 0) {
+                part[0] = sm[g];
+                part[1] = sl[g];
+            }
+#pragma unroll
+            for (int d = 0; d < 4; ++d) part[2 + i + d] = num[d];
+        }
+    }
 }
-// Launch of the merge: quads from 16 splits on, 16 lanes per group from 64
-// (a decode row has only rows x heads x d / 4 groups: 512 at the 0.8B shape,
-// so with one lane or a quad each lane walks many splits in turn).
-int launch_combine(hipStream_t s, const ReadArgs& a) {
-    const long groups = long(a.rows) * a.heads * (a.d / 4);
-    if (a.splits >= 64)
-        hipLaunchKernelGGL(attention_combine_kernel<16>, dim3(ceil_div(groups * 16, 256)), dim3(256), 0, s, a);
-    else if (a.splits >= 16)
-        hipLaunchKernelGGL(attention_combine_kernel<4>, dim3(ceil_div(groups * 4, 256)), dim3(256), 0, s, a);
-    else
-        hipLaunchKernelGGL(attention_combine_kernel<1>, dim3(ceil_div(groups, 256)), dim3(256), 0, s, a);
+
+// Merge the split partials: W waves own one (row, head), a block 4 / W of them
+// (one from W = 4 on). Four dims to a lane, d / 4 lanes (up to 64) to a split's
+// partial: a wave reads whole partials, four steps' loads together, keeps (max,
+// sum, weighted sums) of its own splits, and the lanes of the same dims and the
+// waves are merged by the log-sum-exp rule, in a fixed order. A prefill chunk
+// has rows enough for one wave each; a decode row (8 heads) takes as many waves
+// as give each about four partials. At 8192 positions 6.5 us (13.4 with 16 lanes
+// per 4 dims walking 16 of 256 splits each), 4 shares of 2644 rows 28 us. The partial sums are read as
+// 8-byte pairs (a partial is d + 2 floats).
+template <int W>
+__global__ __launch_bounds__(W < 4 ? 256 : 64 * W) void attention_combine_kernel(ReadArgs a) {
+    typedef float f2v __attribute__((ext_vector_type(2)));
+    constexpr int ROWS = W < 4 ? 4 / W : 1, U = 4;
+    __shared__ float sm[ROWS * W], sd[ROWS * W], sn[ROWS * W][4][64];
+    const int lane = int(threadIdx.x & 63), wb = int(threadIdx.x >> 6), w = wb % W;
+    const int ld = a.d / 4, per = 64 / ld;  // d: a power of two up to 256
+    const int dl = lane % ld, sl = lane / ld;
+    const long rh = long(blockIdx.x) * ROWS + wb / W, total = long(a.rows) * a.heads;  // row * heads + head
+    const int i = 4 * dl;
+    const float* parts = a.parts + size_t(rh < total ? rh : 0) * a.splits * (a.d + 2);
+    float m = -INFINITY, den = 0.f, num[4] = {0.f, 0.f, 0.f, 0.f};
+    auto merge = [&](float mo, float dn, const float (&n)[4]) {
+        const float mn = fmaxf(m, mo);
+        const float c0 = m == -INFINITY ? 0.f : expf(m - mn), c1 = mo == -INFINITY ? 0.f : expf(mo - mn);
+        den = den * c0 + dn * c1;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) num[e] = num[e] * c0 + n[e] * c1;
+        m = mn;
+    };
+    for (int s = w * per + sl; s < a.splits; s += U * W * per) {
+        f2v h[U], lo[U], hi[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const float* p = parts + size_t(min(s + u * W * per, a.splits - 1)) * (a.d + 2);
+            h[u] = *reinterpret_cast<const f2v*>(p);
+            lo[u] = *reinterpret_cast<const f2v*>(p + 2 + i);
+            hi[u] = *reinterpret_cast<const f2v*>(p + 4 + i);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (s + u * W * per < a.splits) merge(h[u].x, h[u].y, {lo[u].x, lo[u].y, hi[u].x, hi[u].y});
+    }
+    for (int o = ld; o < 64; o <<= 1) {  // the lanes of the same dims (both sides form the same value)
+        const float mo = __shfl_xor(m, o, 64), dn = __shfl_xor(den, o, 64);
+        const float n[4] = {__shfl_xor(num[0], o, 64), __shfl_xor(num[1], o, 64), __shfl_xor(num[2], o, 64),
+                            __shfl_xor(num[3], o, 64)};
+        merge(mo, dn, n);
+    }
+    if constexpr (W > 1) {
+        if (sl == 0) {
+            if (dl == 0) {
+                sm[wb] = m;
+                sd[wb] = den;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sn[wb][e][dl] = num[e];
+        }
+        __syncthreads();
+        if (w != 0 || sl != 0) return;
+#pragma unroll
+        for (int v = 1; v < W; ++v) m = fmaxf(m, sm[wb + v]);
+        den = num[0] = num[1] = num[2] = num[3] = 0.f;
+#pragma unroll
+        for (int v = 0; v < W; ++v) {
+            const float c = sm[wb + v] == -INFINITY ? 0.f : expf(sm[wb + v] - m);
+            den += sd[wb + v] * c;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) num[e] += sn[wb + v][e][dl] * c;
+        }
+    } else if (sl != 0) {
+        return;
+    }
+    if (rh >= total) return;
+    const size_t o = size_t(rh) * a.d + i;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) a.out[o + e] = (num[e] / den) * sigmoidf_(a.gate[o + e]);
+}
+template <int W>
+int launch_combine_w(hipStream_t s, const ReadArgs& a) {
+    hipLaunchKernelGGL(attention_combine_kernel<W>, dim3(ceil_div(long(a.rows) * a.heads, W < 4 ? 4 / W : 1)),
+                       dim3(W < 4 ? 256 : 64 * W), 0, s, a);
     return int(hipGetLastError());
+}
+int launch_combine(hipStream_t s, const ReadArgs& a) {
+    const int step = 4 * (256 / a.d);  // splits per wave and round of loads
+    if (a.splits <= step || long(a.rows) * a.heads >= 1024) return launch_combine_w<1>(s, a);
+    if (a.splits <= 2 * step) return launch_combine_w<2>(s, a);
+    if (a.splits <= 4 * step) return launch_combine_w<4>(s, a);
+    if (a.splits <= 8 * step) return launch_combine_w<8>(s, a);
+    return launch_combine_w<16>(s, a);
 }
 
 // ---------------------------------------------------------------- prefill
@@ -780,7 +946,16 @@ int launch_prefill(hipStream_t s, const ReadArgs& a, int group) {
 template <int D>
 int launch_d(hipStream_t s, const ReadArgs& a, int group) {
     dim3 grid(unsigned(a.splits), unsigned(a.kv), unsigned(a.rows));
-    switch (group) {
+    if constexpr (D >= 64) {
+        switch (group) {
+        case 1: hipLaunchKernelGGL((attention_decode_kernel<D, 1>), grid, dim3(256), 0, s, a); break;
+        case 2: hipLaunchKernelGGL((attention_decode_kernel<D, 2>), grid, dim3(256), 0, s, a); break;
+        case 4: hipLaunchKernelGGL((attention_decode_kernel<D, 4>), grid, dim3(256), 0, s, a); break;
+        case 8: hipLaunchKernelGGL((attention_decode_kernel<D, 8>), grid, dim3(256), 0, s, a); break;
+        default: return int(hipErrorInvalidValue);
+        }
+        return int(hipGetLastError());
+    } else switch (group) {
     case 1: hipLaunchKernelGGL((attention_read_kernel<D, 1>), grid, dim3(256), 0, s, a); break;
     case 2: hipLaunchKernelGGL((attention_read_kernel<D, 2>), grid, dim3(256), 0, s, a); break;
     case 4: hipLaunchKernelGGL((attention_read_kernel<D, 4>), grid, dim3(256), 0, s, a); break;
@@ -790,10 +965,12 @@ int launch_d(hipStream_t s, const ReadArgs& a, int group) {
     return int(hipGetLastError());
 }
 
-// Splits for one decode row: about 512 blocks over the KV heads, spans a
-// multiple of 16 positions.
+// Splits for one decode row: about 256 blocks (one per CU) over the KV heads,
+// spans a multiple of 16 positions (at 8192 positions, with 512 blocks the read
+// 10.6 us as with 256, the merge of twice the partials 1 us more; 128 blocks 4 us
+// slower).
 int decode_splits(int length, int kv, int& span) {
-    const int target = 512 / (kv > 0 ? kv : 1);
+    const int target = 256 / (kv > 0 ? kv : 1);
     int s = (length + target - 1) / target;
     s = (s + 15) / 16 * 16;
     if (s < 16) s = 16;
@@ -807,20 +984,23 @@ bool prefill_path(int d, int group, int rows) {
     return rows >= kPrefillMinRows && (d == 64 || d == 128 || d == 256) &&
            (group == 1 || group == 2 || group == 4 || group == 8) && prefill_shape_ok(d, group);
 }
-// KV splits of a prefill chunk: about 512 blocks, at most 8 shares per tile.
-int prefill_splits(int rows, int kv) {
+int prefill_tiles(int length0, int tokens) { return ceil_div(length0 + tokens - 1, 32); }
+// KV splits of a prefill chunk: about 512 blocks, at most kMaxShares shares of at
+// least one tile (128 rows over 2048 positions, kernel + merge: 8 shares 45.8 +
+// 6.6 us, 16 33.4 + 7.3; 12 and 24 in between).
+constexpr int kMaxShares = 16;
+int prefill_splits(int rows, int kv, int tiles) {
     const long blocks = long(ceil_div(rows, 32)) * (kv > 0 ? kv : 1);
-    long s = (512 + blocks - 1) / blocks;
-    return int(s < 1 ? 1 : s > 8 ? 8 : s);
+    const long most = tiles < kMaxShares ? tiles : kMaxShares, s = (512 + blocks - 1) / blocks;
+    return int(s < 1 ? 1 : s > most ? most : s);
 }
 
 // Scratch of a prefill call, in floats: the split partials, then (head dim
 // 256, 4 query heads per KV head) the K and V^T planes at a 256-byte boundary.
-size_t prefill_parts_floats(int tokens, int heads, int kv, int d) {
-    const int splits = prefill_splits(tokens, kv);
+size_t prefill_parts_floats(int tokens, int heads, int kv, int d, int tiles) {
+    const int splits = prefill_splits(tokens, kv, tiles);
     return splits > 1 ? (size_t(tokens) * heads * splits * (d + 2) + 63) / 64 * 64 : 0;
 }
-int prefill_tiles(int length0, int tokens) { return ceil_div(length0 + tokens - 1, 32); }
 
 }  // namespace
 
@@ -829,7 +1009,7 @@ size_t attention_scratch_needed(const Params& a) {
     const int group = a.n[2] > 0 ? a.n[1] / a.n[2] : 0;
     if (tokens > 1) {
         if (!prefill_path(a.n[0], group, tokens)) return 0;
-        size_t need = prefill_parts_floats(tokens, a.n[1], a.n[2], a.n[0]);
+        size_t need = prefill_parts_floats(tokens, a.n[1], a.n[2], a.n[0], prefill_tiles(a.n[3], tokens));
         if (a.n[0] == 256 && group == 4)
             need += size_t(a.n[2]) * prefill_tiles(a.n[3], tokens) * (B3_KBLK + B3_VBLK) / sizeof(float);
         return need;
@@ -864,12 +1044,13 @@ int run_attention_read(hipStream_t s, int heads_count, const Params& p, float* s
         a.span = a.length0 + a.rows;  // row r reads its own length inside the span
     }
     if (prefill_path(a.d, group, a.rows)) {
-        a.splits = prefill_splits(a.rows, a.kv);
-        const size_t parts = prefill_parts_floats(a.rows, a.heads, a.kv, a.d);
+        const int tiles = prefill_tiles(a.length0, a.rows);
+        a.splits = prefill_splits(a.rows, a.kv, tiles);
+        const size_t parts = prefill_parts_floats(a.rows, a.heads, a.kv, a.d, tiles);
         if (parts > scratch_len) return int(hipErrorInvalidValue);
         if (a.splits > 1) a.parts = scratch;
         if (a.d == 256 && group == 4) {
-            a.tiles = prefill_tiles(a.length0, a.rows);
+            a.tiles = tiles;
             const size_t planes = size_t(a.kv) * a.tiles * (B3_KBLK + B3_VBLK) / sizeof(float);
             if (parts + planes > scratch_len) return int(hipErrorInvalidValue);
             a.kpl = reinterpret_cast<char*>(scratch + parts);

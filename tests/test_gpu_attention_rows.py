@@ -1,0 +1,63 @@
+"""One decode row of AttentionRead (op 10) at the edges of its chunks, spans and
+merges, for every head dim and group size of the decode kernels, and a prefill
+chunk's KV shares, against the CPU op."""
+import numpy as np
+import pytest
+
+from bridges import rnd
+from conftest import ROOT
+from parity import parity
+from qwen_mi355x.bridge import Bridge
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def both():
+    g, c = Bridge(), Bridge(ROOT / "oracle" / "lib" / "libqwen_ops_bridge.so", kind=0)
+    yield g, c
+    g.close()
+    c.close()
+
+
+def read(br, d, heads, kv, length, rows, data):
+    q, k, v, gate = (br.upload(x) for x in data)
+    out = br.alloc(rows * heads * d)
+    scores = br.alloc(heads * max(length + rows, 16 * (d + 2)))
+    br.run("ATTENTION_READ", heads, [out, q, k, v, gate, scores],
+           [d, heads, kv, length, length + rows, rows, scores.n // heads])
+    return out.read()
+
+
+@pytest.mark.parametrize("d,heads,kv", [(256, 8, 2), (256, 8, 1), (256, 2, 1), (256, 2, 2), (128, 8, 2), (128, 3, 3),
+                                        (128, 8, 1), (64, 4, 2), (64, 8, 1), (64, 4, 1), (32, 4, 1), (16, 4, 2)])
+@pytest.mark.parametrize("length", [1, 15, 32, 33, 65, 512, 2049, 4111])
+def test_decode_row(both, d, heads, kv, length):
+    print(f"decode row d={d} heads={heads}/{kv} length={length}", flush=True)
+    rng = np.random.default_rng(d + heads + length)
+    data = [rnd(rng, heads * d), rnd(rng, length * kv * d), rnd(rng, length * kv * d), rnd(rng, heads * d)]
+    got, want = (read(b, d, heads, kv, length, 1, data) for b in both)
+    parity(got, want, where=f"decode row {d} {heads}/{kv} {length}")
+
+
+@pytest.mark.parametrize("length,rows", [(1, 9), (1, 33), (30, 40), (500, 32), (513, 17), (1000, 65)])
+def test_shares(both, length, rows):
+    """KV shares from one tile each up to the most, rows past a 32-row tile."""
+    print(f"shares length={length} rows={rows}", flush=True)
+    d, heads, kv = 256, 8, 2
+    rng = np.random.default_rng(length + rows)
+    n = length + rows
+    data = [rnd(rng, rows * heads * d), rnd(rng, n * kv * d), rnd(rng, n * kv * d), rnd(rng, rows * heads * d)]
+    got, want = (read(b, d, heads, kv, length, rows, data) for b in both)
+    parity(got, want, where=f"shares {length} {rows}")
+
+
+def test_large_scores(both):
+    """Scores of hundreds (one position takes all the weight) and equal scores."""
+    d, heads, kv, length = 256, 8, 2, 300
+    rng = np.random.default_rng(0)
+    for scale in (30.0, 0.0):
+        data = [rnd(rng, heads * d) * np.float32(scale), rnd(rng, length * kv * d), rnd(rng, length * kv * d),
+                rnd(rng, heads * d)]
+        got, want = (read(b, d, heads, kv, length, 1, data) for b in both)
+        parity(got, want, where=f"scale {scale}")
