@@ -27,11 +27,11 @@
 // Measured (one call, weights cold, launch included; before: the prefill GEMM
 // of gemm_p3.hip over planes, or gemm_bf3_kernel under 64 tokens and for
 // matrices without planes):
-//   GLU 2 x 3584 x 1024, fp32 planes: 23 tokens 70.2 -> 14.2 us, 128 tokens 25.1 -> 17.3
-//   GLU, BF16 plane: 23 tokens 54.1 -> 7.2 us, 128 tokens 25.1 -> 11.2, 512 tokens 38.3 -> 29.6
-//   GLU, int8 without a plane, 128 tokens: 59.5 -> 12.6 us
-//   down 1024 x 3584, fp32 planes: 23 tokens 24.8 -> 12.1 us, 128 tokens 22.2 -> 12.9
-//   q|k|v 5120 x 1024, 128 tokens: fp32 planes 17.2 -> 12.3 us, BF16 19.4 -> 9.6
+//   GLU 2 x 3584 x 1024, fp32 planes: 23 tokens 70.1 -> 13.7 us, 128 tokens 25.3 -> 16.9
+//   GLU, BF16 plane: 23 tokens 54.1 -> 7.1 us, 128 tokens 22.7 -> 10.3, 512 tokens 38.0 -> 28.5
+//   GLU, int8 without a plane, 128 tokens: 59.5 -> 12.3 us
+//   down 1024 x 3584, fp32 planes: 23 tokens 24.7 -> 12.0 us, 128 tokens 22.0 -> 12.8
+//   q|k|v 5120 x 1024, 128 tokens: fp32 planes 17.1 -> 12.0 us, BF16 19.4 -> 8.6
 #include <type_traits>
 
 #include "common.h"
@@ -104,6 +104,11 @@ __device__ __forceinline__ void wload(WReg<T, RAW>& r, const char* p) {
         for (int q = 0; q < kPlanes<T>; ++q) r.h[q] = *reinterpret_cast<const bf16x8*>(p + 1024 * q);
     }
 }
+// Plane q alone (planes only).
+template <WeightType T>
+__device__ __forceinline__ void wload_plane(WReg<T, false>& r, const char* p, int q) {
+    r.h[q] = *reinterpret_cast<const bf16x8*>(p + 1024 * q);
+}
 template <WeightType T, bool RAW>
 __device__ __forceinline__ void wplanes(const WReg<T, RAW>& r, bf16x8 (&h)[kPlanes<T>]) {
     if constexpr (RAW && T == WeightType::F32) {
@@ -124,45 +129,53 @@ __device__ __forceinline__ void wplanes(const WReg<T, RAW>& r, bf16x8 (&h)[kPlan
 template <WeightType T>
 constexpr int kRawBytes = T == WeightType::F32 ? 4 : T == WeightType::BF16 ? 2 : 1;
 
-// The part products of one X operand (three planes) and one W operand, smallest first.
-template <WeightType T, class F>
-__device__ __forceinline__ void products(F&& mfma) {
-    if constexpr (T == WeightType::F32) {
-        constexpr int P[6] = {2, 1, 0, 1, 0, 0}, Q[6] = {0, 1, 2, 0, 1, 0};
-#pragma unroll
-        for (int q = 0; q < 6; ++q) mfma(P[q], Q[q]);
-    } else {
-#pragma unroll
-        for (int q = 2; q >= 0; --q) mfma(q, 0);
-    }
-}
+// The part products of an X operand (three planes) and a W operand, from the
+// smallest: product q is x_P(q) w_Q(q), after which plane xdead(q) of X and
+// wdead(q) of W (-1: none) are not used again in the step.
+template <WeightType T>
+struct Products {
+    static constexpr int N = 3;
+    static constexpr int P(int q) { return 2 - q; }
+    static constexpr int Q(int) { return 0; }
+    static constexpr int xdead(int q) { return 2 - q; }
+    static constexpr int wdead(int q) { return q == 2 ? 0 : -1; }
+};
+template <>
+struct Products<WeightType::F32> {
+    static constexpr int N = 6;
+    static constexpr int P(int q) { return q == 0 ? 2 : q < 3 ? 1 : 0; }
+    static constexpr int Q(int q) { return q == 1 || q == 4 ? 1 : q == 3 ? 2 : 0; }
+    static constexpr int xdead(int q) { return q == 0 ? 2 : q == 2 ? 1 : q == 5 ? 0 : -1; }
+    static constexpr int wdead(int q) { return q < 3 ? -1 : 5 - q; }
+};
 
-// n steps through a ring of NS (even) register buffers: load(buffer, step) NS
-// steps ahead of multiply(buffer, step % 2). The main loop's loads are unconditional (a join
-// between a path with loads and one without would make the compiler wait for
-// more than the buffer it needs).
-template <int NS, class Buf, class L, class M>
-__device__ __forceinline__ void ring(int n, L&& load, M&& multiply) {
+// n steps through a ring of NS (even) register buffers. step(buffer, step % 2,
+// next) multiplies a buffer and, for next >= 0, loads step `next` into it plane
+// by plane as the products are done with it: loads issued in a burst after the
+// products stall the wave (the CU's vector memory path takes 16 clocks per KiB
+// and a wave issues in order), among them they do not: q|k|v of 128 fp32 tokens
+// 14.5 -> 12.0 us, of 300 25.8 -> 20.7, the BF16 GLU of 128 tokens 11.4 -> 10.3. The main loop's
+// loads are unconditional (a join between a path with loads and one without
+// would make the compiler wait for more than the buffer it needs).
+template <int NS, class Buf, class L, class S>
+__device__ __forceinline__ void ring(int n, L&& load, S&& step) {
     Buf b[NS];
 #pragma unroll
     for (int i = 0; i < NS; ++i) load(b[i], min(i, n - 1));
     int s = 0;
     for (; s + 2 * NS <= n; s += NS)
 #pragma unroll
-        for (int i = 0; i < NS; ++i) {
-            multiply(b[i], i % 2);
-            load(b[i], s + i + NS);
-        }
+        for (int i = 0; i < NS; ++i) step(b[i], i % 2, s + i + NS);
 #pragma unroll
     for (int i = 0; i < NS; ++i)
         if (s + i < n) {
-            multiply(b[i], i % 2);
+            step(b[i], i % 2, -1);
             if (s + i + NS < n) load(b[i], s + i + NS);
         }
     s += NS;
 #pragma unroll
     for (int i = 0; i < NS - 1; ++i)
-        if (s + i < n) multiply(b[i], i % 2);
+        if (s + i < n) step(b[i], i % 2, -1);
 }
 
 // Wave w's k tiles (w, w + NW, ...) of a (32 TMT) x (32 TNT) tile into acc. xb
@@ -175,7 +188,8 @@ __device__ __forceinline__ void k_wave(f16v (&acc)[TMT][TNT], const char* const 
                                        int kt, int w) {
     constexpr int XSTEP = 3 * 1024, WSTEP = RAW ? 16 * kRawBytes<T> : kPlanes<T> * 1024;
     const int n = (kt - w + NW - 1) / NW;
-    constexpr int NS = TMT * TNT == 4 ? 2 : 4;  // buffers that fit 256 VGPRs
+    // buffers that fit 256 VGPRs
+    constexpr int NS = TMT * TNT == 4 || (T == WeightType::F32 && TMT == 1 && TNT == 2) ? 2 : 4;
     struct Buf {
         bf16x8 x[TMT][3];
         WReg<T, RAW> w[TNT];
@@ -196,21 +210,42 @@ __device__ __forceinline__ void k_wave(f16v (&acc)[TMT][TNT], const char* const 
         for (int j = 0; j < TNT; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = odd[i][j][r] = 0.f;
-    auto multiply = [&](const Buf& b, int parity) {
+    auto step = [&](Buf& b, int parity, int next) {
+        using Pr = Products<T>;
+        const size_t k = size_t(w + NW * next);
         bf16x8 h[TNT][kPlanes<T>];
 #pragma unroll
         for (int j = 0; j < TNT; ++j) wplanes<T, RAW>(b.w[j], h[j]);
-        products<T>([&](int px, int pw) {
+        if (RAW && next >= 0) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < TNT; ++j) wload<T, RAW>(b.w[j], wb[j] + k * WSTEP);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int q = 0; q < Pr::N; ++q) {
 #pragma unroll
             for (int i = 0; i < TMT; ++i)
 #pragma unroll
                 for (int j = 0; j < TNT; ++j) {
                     f16v& a = parity ? odd[i][j] : acc[i][j];
-                    a = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.x[i][px], h[j][pw], a, 0, 0, 0);
+                    a = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.x[i][Pr::P(q)], h[j][Pr::Q(q)], a, 0, 0, 0);
                 }
-        });
+            if (next < 0) continue;
+            __builtin_amdgcn_sched_barrier(0);
+            if (Pr::xdead(q) >= 0)
+#pragma unroll
+                for (int i = 0; i < TMT; ++i)
+                    b.x[i][Pr::xdead(q)] =
+                        *reinterpret_cast<const bf16x8*>(xb[i] + k * XSTEP + 1024 * Pr::xdead(q));
+            if constexpr (!RAW)
+                if (Pr::wdead(q) >= 0)
+#pragma unroll
+                    for (int j = 0; j < TNT; ++j) wload_plane<T>(b.w[j], wb[j] + k * WSTEP, Pr::wdead(q));
+            __builtin_amdgcn_sched_barrier(0);
+        }
     };
-    if (w < kt) ring<NS, Buf>(n, load, multiply);
+    if (w < kt) ring<NS, Buf>(n, load, step);
 #pragma unroll
     for (int i = 0; i < TMT; ++i)
 #pragma unroll
@@ -383,17 +418,35 @@ __global__ __launch_bounds__(64 * NW) void kw_narrow_kernel(KwArgs p) {
                 for (int q = 0; q < 3; ++q)
                     b.x[i][q] = *reinterpret_cast<const bf16x8*>(xb + s * 6144 + 1024 * q + 256 * i);
         };
-        auto multiply = [&](const Buf& b, int parity) {
+        auto step = [&](Buf& b, int parity, int next) {
+            using Pr = Products<T>;
+            const size_t s = size_t(w + NW * next);
             bf16x8 h[WP];
             wplanes<T, RAW>(b.w, h);
-            products<T>([&](int px, int pw) {
+            if (RAW && next >= 0) {
+                __builtin_amdgcn_sched_barrier(0);
+                wload<T, RAW>(b.w, wb + s * WSTEP);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int q = 0; q < Pr::N; ++q) {
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
-                    acc[i][parity] =
-                        __builtin_amdgcn_mfma_f32_16x16x32_bf16(b.x[i][px], h[pw], acc[i][parity], 0, 0, 0);
-            });
+                    acc[i][parity] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b.x[i][Pr::P(q)], h[Pr::Q(q)],
+                                                                            acc[i][parity], 0, 0, 0);
+                if (next < 0) continue;
+                __builtin_amdgcn_sched_barrier(0);
+                if (Pr::xdead(q) >= 0)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+                        b.x[i][Pr::xdead(q)] =
+                            *reinterpret_cast<const bf16x8*>(xb + s * 6144 + 1024 * Pr::xdead(q) + 256 * i);
+                if constexpr (!RAW)
+                    if (Pr::wdead(q) >= 0) wload_plane<T>(b.w, wb + s * WSTEP, Pr::wdead(q));
+                __builtin_amdgcn_sched_barrier(0);
+            }
         };
-        if (w < steps) ring<4, Buf>((steps - w + NW - 1) / NW, load, multiply);
+        if (w < steps) ring<4, Buf>((steps - w + NW - 1) / NW, load, step);
     };
     if (it.raw) {
         const int row = min(n0 + (lane & 15), it.rows - 1);
@@ -473,10 +526,10 @@ Tile pick_tile(WeightType t, const KwItem* items, int n, int M) {
 
 // Up to kKwMaxTokens tokens, and while the 64 x 64 tiles number at most 640
 // (three planes; against the prefill GEMM's 128 x 256 tiles: 560 of the GLU at
-// 300 tokens 38.8 against 42.3 us, 640 of q|k|v at 512 tokens 35.9 against
-// 40.2, 1024 of 8192 rows at 512 tokens 62 against 49) or 1152 (one plane, or
-// no planes at all: 896 of the GLU at 512 tokens 29.6 against 38.3 us; 1792 of
-// them at 1024 tokens 82 against 57).
+// 300 tokens 35.1 against 41.9 us, 640 of q|k|v at 512 tokens 31.1 against
+// 39.7, 1024 of 8192 rows at 512 tokens 54 against 48) or 1152 (one plane, or
+// no planes at all: 896 of the GLU at 512 tokens 28.5 against 38.0 us; with
+// one accumulator chain and burst loads 1792 of them took 82 against 57).
 bool kw_wanted(WeightType t, bool raw, int M, int rows) {
     const long tiles = long(ceil_div(M, 64)) * long(ceil_div(rows, 64));
     return M <= kKwMaxTokens && (M <= 64 || tiles <= (t == WeightType::F32 && !raw ? 640 : 1152));
@@ -511,7 +564,7 @@ int kw_glu(hipStream_t s, WeightType t, float* product, __bf16* planes, const Kw
         (reinterpret_cast<uintptr_t>(product) | reinterpret_cast<uintptr_t>(gate.scale) |
          reinterpret_cast<uintptr_t>(up.scale)) % 16)
         return int(hipErrorInvalidValue);
-    // one plane: 32-token tiles also past one round of 64-token ones (300 tokens 25 against 29 us)
+    // one plane: 32-token tiles also past one round of 64-token ones (300 tokens 25 against 29 us with burst loads)
     const long cols = gate.rows / 32, small = cols * ceil_div(M, 32), large = cols * ceil_div(M, 64);
     const Tile tile = small <= 256 || (large > 256 && t != WeightType::F32 && !gate.raw) ? k32x64 : k64x64;
     KwArgs a{};
