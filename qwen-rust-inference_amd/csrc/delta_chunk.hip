@@ -52,18 +52,25 @@ typedef float f4v __attribute__((ext_vector_type(4)));
 constexpr int kPrep = 512;              // threads of a prep block (8 waves)
 constexpr int kPrepLoads = kC * kD / 4 / kPrep;  // float4 of q (of k, of V) per thread
 
+// 79 KB of LDS, so that two blocks share a CU (128 VGPRs a wave, 4 waves per
+// SIMD): one block's loads, exponentials and serial inversion run beside the
+// other's MFMAs. A block's time is a chain of phases, none bound by the whole
+// CU; with A and L whole in LDS (one block per CU) 2644 tokens of the 0.8B shape
+// (672 tasks) took 70 us a layer, now 54, and 128 tokens (32 tasks) 19 us, now 17.
 struct PrepLds {
     // row stride 132 (4 mod 64 banks): the Gram products' MFMA operand reads
     // (16 rows x 4 interleaved k per step) hit 64 distinct banks
-    float ks[kC][kD + 4], qs[kC][kD + 4];
-    // am holds A transposed: am[s][t] = A_ts (s < t), so the solve's column
-    // sweeps read rows
-    float am[kC][kC + 4], lm[kC][kC + 4];
-    // inverses of the four 16 x 16 diagonal blocks of I + A: li[i][t][s] = ((I + A)_ii^-1)_ts
-    float li[kC / 16][16][16];
+    alignas(16) float ks[kC][kD + 4], qs[kC][kD + 4];
+    // The lower 16 x 16 tiles of A, each transposed, then the inverses of the
+    // diagonal blocks of I + A in the place of A's. Tile (i, j) is
+    // am[lower(i, j)]: entry 16 s + t is A of row 16 i + t and column 16 j + s
+    // (0 for s >= t on the diagonal); an inverse's entry 16 t + s its (t, s).
+    // The tile stride puts the diagonal tiles in different banks.
+    alignas(16) float am[10][16 * 16 + 4];
     double gd[kC];
     float bs[kC], eg[kC], el[kC];
 };
+constexpr int lower(int i, int j) { return i * (i + 1) / 2 + j; }
 
 // The record of chunk c0 + xi of head h, into slot xi of `scratch`; every
 // thread of a kPrep-thread block takes part.
@@ -72,8 +79,6 @@ __device__ __forceinline__ void prep_task(const Params& a, int gated, int qkn, i
     auto& ks = P.ks;
     auto& qs = P.qs;
     auto& am = P.am;
-    auto& lm = P.lm;
-    auto& li = P.li;
     auto& gd = P.gd;
     auto& bs = P.bs;
     auto& eg = P.eg;
@@ -176,12 +181,7 @@ __device__ __forceinline__ void prep_task(const Params& a, int gated, int qkn, i
     }
     __syncthreads();
     {  // Gram products K K^T and Q K^T on MFMA, the 10 lower 16 x 16 tiles (sj <= ti)
-        const int w = tid >> 6, l = tid & 63, lc = l & 15, q = l >> 4;
-        for (int e = tid; e < 6 * 256; e += kPrep) {  // the upper tiles are zero
-            const int tile = e >> 8, ti = tile < 3 ? 0 : tile < 5 ? 1 : 2, sj = tile < 3 ? tile + 1 : tile < 5 ? tile - 1 : 3;
-            const int t = 16 * ti + ((e >> 4) & 15), s2 = 16 * sj + (e & 15);
-            lm[t][s2] = 0.f;
-        }
+        const int w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, lc = l & 15, q = l >> 4;
         // the 20 products (tile j of the list (ti, sj) = (0,0) (1,0) (1,1) (2,0) ... (3,3), K K^T
         // or Q K^T) dealt to the 8 waves: product w + 8 k
         for (int pr = w; pr < 20; pr += kPrep / 64) {
@@ -189,15 +189,19 @@ __device__ __forceinline__ void prep_task(const Params& a, int gated, int qkn, i
             const int ti = j < 1 ? 0 : j < 3 ? 1 : j < 6 ? 2 : 3, sj = j - ti * (ti + 1) / 2;
             // MFMA step 4 m + e, lane (lc, q) takes k = 32 q + 4 m + e: a lane's operands of a
             // tile are 8 contiguous float4 per matrix, read before the 32 MFMAs
-            float (*as)[kD + 4] = qk ? qs : ks;
+            // K K^T as rows t, columns s; Q K^T transposed (rows s, columns t), so that a lane's
+            // four values go to four 256-byte runs of the record's L (its tiles past the diagonal
+            // are neither written nor used)
+            const float* pa = &ks[16 * (qk ? sj : ti) + lc][32 * q];
+            const float* pb = qk ? &qs[16 * ti + lc][32 * q] : &ks[16 * sj + lc][32 * q];
             // two independent accumulator chains (k below and above 64 within each lane group's
             // 32), added at the end
             f4v acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
             f4v xa[8], xb[8];
 #pragma unroll
             for (int m = 0; m < 8; ++m) {
-                xa[m] = *reinterpret_cast<const f4v*>(&as[16 * ti + lc][32 * q + 4 * m]);
-                xb[m] = *reinterpret_cast<const f4v*>(&ks[16 * sj + lc][32 * q + 4 * m]);
+                xa[m] = *reinterpret_cast<const f4v*>(pa + 4 * m);
+                xb[m] = *reinterpret_cast<const f4v*>(pb + 4 * m);
             }
 #pragma unroll
             for (int m = 0; m < 4; ++m)
@@ -207,48 +211,59 @@ __device__ __forceinline__ void prep_task(const Params& a, int gated, int qkn, i
                     acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[m + 4][e], xb[m + 4][e], acc1, 0, 0, 0);
                 }
             const f4v acc = acc0 + acc1;
+            if (qk) {
+                const int t = 16 * ti + lc;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int t = 16 * ti + 4 * q + r, s2 = 16 * sj + lc;
-                const float e = s2 <= t ? expf(float(gd[t] - gd[s2])) : 0.f;
-                if (qk)
-                    lm[t][s2] = e * acc[r];
-                else
-                    am[s2][t] = s2 < t ? bs[t] * e * acc[r] : 0.f;
+                for (int r = 0; r < 4; ++r) {  // element q of float4 (ti, m = sj, lane lc + 16 r)
+                    const int s2 = 16 * sj + 4 * q + r;
+                    const float e = s2 <= t ? expf(float(gd[t] - gd[s2])) : 0.f;
+                    rec[kL + (ti * 256 + sj * 64 + 16 * r + lc) * 4 + q] = e * acc[r];
+                }
+            } else {
+                const int s2 = 16 * sj + lc;
+                f4v v;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int t = 16 * ti + 4 * q + r;
+                    const float e = s2 <= t ? expf(float(gd[t] - gd[s2])) : 0.f;
+                    v[r] = s2 < t ? bs[t] * e * acc[r] : 0.f;
+                }
+                *reinterpret_cast<f4v*>(&am[j][16 * lc + 4 * q]) = v;
             }
         }
     }
     __syncthreads();
-    // e^G Q, (e^{G_63-G} K)^T and L into the record, one float4 of the
-    // destination per thread step (contiguous stores)
-    for (int d = tid; d < kC * kD / 4; d += kPrep) {
-        const int l = d & 63, lr = l & 15, q = l >> 4;
-        {  // e^G Q: 4 tiles of 16 rows, K = 128 (8 float4 per lane)
-            const int tile = d >> 9, m = (d >> 6) & 7, t = tile * 16 + lr, k = 16 * m + q;
-            rec4[kQ / 4 + d] = f4v{qs[t][k], qs[t][k + 4], qs[t][k + 8], qs[t][k + 12]} * eg[t];
+    // The last wave inverts the diagonal blocks; the others meanwhile write e^G Q
+    // and (e^{G_63-G} K)^T into the record, one float4 of the destination per
+    // thread step (contiguous stores). The inversion is a serial chain of 15 steps:
+    // after the wave's share of the record it was the phase's critical path.
+    if (tid < kPrep - 64) {
+        for (int d = tid; d < kC * kD / 4; d += kPrep - 64) {
+            const int l = d & 63, lr = l & 15, q = l >> 4;
+            {  // e^G Q: 4 tiles of 16 rows, K = 128 (8 float4 per lane)
+                const int tile = d >> 9, m = (d >> 6) & 7, t = tile * 16 + lr, k = 16 * m + q;
+                rec4[kQ / 4 + d] = f4v{qs[t][k], qs[t][k + 4], qs[t][k + 8], qs[t][k + 12]} * eg[t];
+            }
+            {  // (e^{G_63-G} K)^T: 8 tiles of 16 key dims, K = 64 tokens (4 float4 per lane)
+                const int tile = d >> 8, m = (d >> 6) & 3, i = tile * 16 + lr, t = 16 * m + q;
+                rec4[kK / 4 + d] = f4v{el[t] * ks[t][i], el[t + 4] * ks[t + 4][i], el[t + 8] * ks[t + 8][i],
+                                       el[t + 12] * ks[t + 12][i]};
+            }
         }
-        {  // (e^{G_63-G} K)^T: 8 tiles of 16 key dims, K = 64 tokens (4 float4 per lane)
-            const int tile = d >> 8, m = (d >> 6) & 3, i = tile * 16 + lr, t = 16 * m + q;
-            rec4[kK / 4 + d] = f4v{el[t] * ks[t][i], el[t + 4] * ks[t + 4][i], el[t + 8] * ks[t + 8][i],
-                                   el[t + 12] * ks[t + 12][i]};
-        }
-        if (d < kC * kC / 4) {  // L: 4 tiles of 16 tokens, K = 64 tokens
-            const int tile = d >> 8, m = (d >> 6) & 3, t = tile * 16 + lr, k = 16 * m + q;
-            rec4[kL / 4 + d] = f4v{lm[t][k], lm[t][k + 4], lm[t][k + 8], lm[t][k + 12]};
-        }
-    }
-    if (tid >= kPrep - 64) {  // the last wave: lane (i, j) = column j of the inverse of diagonal block i,
-                              // by forward substitution (y_t = [t == j] - A_t0 y_0 - ..., in that order)
-        const int i = (tid & 63) >> 4, j = tid & 15, o = 16 * i;
+    } else {  // lane (i, j) = column j of the inverse of diagonal block i, by forward
+              // substitution (y_t = [t == j] - A_t0 y_0 - ..., in that order)
+        const int i = (tid & 63) >> 4, j = tid & 15;
+        float* const tile = am[lower(i, i)];
         float y[16];
 #pragma unroll
         for (int t = 0; t < 16; ++t) y[t] = t == j ? 1.f : 0.f;
 #pragma unroll
         for (int s2 = 0; s2 < 15; ++s2)
 #pragma unroll
-            for (int t = s2 + 1; t < 16; ++t) y[t] = fmaf(-am[o + s2][o + t], y[s2], y[t]);
+            for (int t = s2 + 1; t < 16; ++t) y[t] = fmaf(-tile[16 * s2 + t], y[s2], y[t]);
+        __builtin_amdgcn_wave_barrier();  // the wave's reads of the block before its inverse (LDS is in order)
 #pragma unroll
-        for (int t = 0; t < 16; ++t) li[i][t][j] = y[t];
+        for (int t = 0; t < 16; ++t) tile[16 * t + j] = y[t];
     }
     __syncthreads();
     {  // right-hand sides: beta e^G K in ks, beta V in qs
@@ -279,13 +294,14 @@ __device__ __forceinline__ void prep_task(const Params& a, int gated, int qkn, i
                 f4v acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int st = 0; st < 4 * i; ++st) {
-                    const int k = 4 * st + q;  // A[16 i + lc][k] = am[k][16 i + lc]
-                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(am[k][16 * i + lc], base[k * RS + lc], acc, 0, 0, 0);
+                    const int k = 4 * st + q;  // A[16 i + lc][k]
+                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(am[lower(i, st / 4)][16 * (k & 15) + lc],
+                                                               base[k * RS + lc], acc, 0, 0, 0);
                 }
                 f4v b;  // B_i - A X: row 16 i + 4 q + r, column lc
 #pragma unroll
                 for (int r = 0; r < 4; ++r) b[r] = base[(16 * i + 4 * q + r) * RS + lc] - acc[r];
-                const f4v inv = *reinterpret_cast<const f4v*>(&li[i][lc][4 * q]);  // row lc, k = 4 q + st
+                const f4v inv = *reinterpret_cast<const f4v*>(&am[lower(i, i)][16 * lc + 4 * q]);  // row lc, k = 4 q + st
                 f4v x = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int st = 0; st < 4; ++st) x = __builtin_amdgcn_mfma_f32_16x16x4f32(inv[st], b[st], x, 0, 0, 0);
@@ -309,7 +325,7 @@ __device__ __forceinline__ void prep_task(const Params& a, int gated, int qkn, i
     if (tid == 0) rec[kG] = eg[kC - 1];
 }
 
-__global__ __launch_bounds__(kPrep) void rule_chunk_prep_kernel(Params a, int gated, int qkn, int c0, float* scratch) {
+__global__ __launch_bounds__(kPrep) __attribute__((amdgpu_waves_per_eu(4))) void rule_chunk_prep_kernel(Params a, int gated, int qkn, int c0, float* scratch) {
     __shared__ PrepLds P;
     prep_task(a, gated, qkn, c0, scratch, int(blockIdx.x), int(blockIdx.y), P);
 }
@@ -489,7 +505,7 @@ __global__ __launch_bounds__(256) void rule_chunk_scan_kernel(Params a, int c0, 
 // on 4 of their 8 waves); the others make the records of the next group's
 // chunks [pc0, pc0 + pchunks) into `prec`, the (chunk, head) tasks dealt
 // round-robin. The two record buffers are disjoint and neither job waits for
-// the other. Their LDS together (~122 KiB) leaves room for one block per CU,
+// the other. Their LDS together (92 KiB) leaves room for one block per CU,
 // so on an idle device the blocks take one CU each and the prep work never
 // shares a CU with the latency-bound scan.
 __global__ __launch_bounds__(kPrep) void rule_chunk_scan_prep_kernel(Params a, int gated, int qkn, int nscan, int sc0,
