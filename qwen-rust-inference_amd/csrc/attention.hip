@@ -739,8 +739,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __shared__ __attribute__((aligned(16))) __bf16 ks[B3_KBLK / 2];  // [3][32][B3_KROW] + DMA padding
     __shared__ __attribute__((aligned(16))) __bf16 vt[B3_VBLK / 2];  // [3][D][B3_VROW] + DMA padding
     __shared__ float xch[8][16][64];
-    const int qtiles = (a.rows + 31) / 32;
-    const int q0 = (qtiles - 1 - int(blockIdx.x)) * 32, kvh = blockIdx.y;  // longest rows first
+    // the blocks of the longest rows first, over all shares and KV heads: with the shares
+    // outermost the last ones dispatched were long again (2644 tokens: a 42-tile schedule, now 31)
+    const int q0 = int(gridDim.y - 1 - blockIdx.y) * 32, kvh = int(blockIdx.x) % a.kv, z = int(blockIdx.x) / a.kv;
     const int tid = int(threadIdx.x), lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), lc = lane & 31,
               hl = lane >> 5;
     const int g = w & 3, dh = w >> 2, d0 = dh * HALF;
@@ -748,10 +749,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int len = a.length0 + qrow;  // positions [0, len) visible to this lane's query
     const int len_max = a.length0 + min(a.rows, q0 + 32) - 1;
     const int all_tiles = (len_max + 31) / 32, share = (all_tiles + a.splits - 1) / a.splits;
-    const int t_begin = int(blockIdx.z) * share, t_end = min(all_tiles, t_begin + share);
+    const int t_begin = z * share, t_end = min(all_tiles, t_begin + share);
     if (t_begin >= t_end) {  // an empty share (early query tiles): a neutral partial
         if (qrow < a.rows && dh == 0) {
-            float* part = a.parts + ((size_t(qrow) * a.heads + head) * a.splits + blockIdx.z) * (D + 2);
+            float* part = a.parts + ((size_t(qrow) * a.heads + head) * a.splits + z) * (D + 2);
             for (int i = hl; i < D + 2; i += 2) part[i] = i == 0 ? -INFINITY : 0.f;
         }
         return;
@@ -904,7 +905,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 a.out[idx] = (o[dt][r] / den) * sigmoidf_(a.gate[idx]);
             }
     } else if (qrow < a.rows) {
-        float* part = a.parts + ((size_t(qrow) * a.heads + head) * a.splits + blockIdx.z) * (D + 2);
+        float* part = a.parts + ((size_t(qrow) * a.heads + head) * a.splits + z) * (D + 2);
         if (hl == 0 && dh == 0) {
             part[0] = m;
             part[1] = den;
@@ -923,7 +924,8 @@ int launch_prefill_g(hipStream_t s, const ReadArgs& a) {
         if constexpr (D == 256 && G == 4) {
             hipLaunchKernelGGL(kv_planes_kernel, dim3(unsigned(a.tiles), unsigned(a.kv)), dim3(256), 0, s, a,
                                a.length0 + a.rows - 1);
-            hipLaunchKernelGGL(attention_prefill_bf3_kernel, grid, dim3(512), 0, s, a);
+            hipLaunchKernelGGL(attention_prefill_bf3_kernel, dim3(unsigned(a.kv * a.splits), ceil_div(a.rows, 32)),
+                               dim3(512), 0, s, a);
         } else
             hipLaunchKernelGGL((attention_prefill_kernel<D, G>), grid, dim3(64 * G), 0, s, a);
         if (a.splits == 1) return int(hipGetLastError());
@@ -978,18 +980,52 @@ int decode_splits(int length, int kv, int& span) {
     return (length + s - 1) / s;
 }
 
-constexpr int kPrefillMinRows = 8;  // fewer rows (decode, verify): attention_read_kernel
+constexpr int kPrefillMinRows = 8;  // fewer rows (decode, verify): attention_decode_kernel, attention_read_kernel
 
 bool prefill_path(int d, int group, int rows) {
     return rows >= kPrefillMinRows && (d == 64 || d == 128 || d == 256) &&
            (group == 1 || group == 2 || group == 4 || group == 8) && prefill_shape_ok(d, group);
 }
 int prefill_tiles(int length0, int tokens) { return ceil_div(length0 + tokens - 1, 32); }
-// KV splits of a prefill chunk: about 512 blocks, at most kMaxShares shares of at
-// least one tile (128 rows over 2048 positions, kernel + merge: 8 shares 45.8 +
-// 6.6 us, 16 33.4 + 7.3; 12 and 24 in between).
+// KV splits of a prefill chunk: at most kMaxShares shares of at least one tile.
 constexpr int kMaxShares = 16;
-int prefill_splits(int rows, int kv, int tiles) {
+bool bf3_shape(int d, int heads, int kv) { return d == 256 && kv > 0 && heads == 4 * kv; }
+// attention_prefill_bf3_kernel runs one block per CU, longest first: the
+// schedule's length in tiles (5.4 us each), a block taking its share plus 1.5,
+// is at least the longest block, the mean per CU, and j times block 256 (j - 1)
+// + 1 (so many CUs hold j blocks at least as long as it); then the partials'
+// way through memory (5 TB/s) and the merge's launch. The smallest over the
+// shares is taken: within 3 % of the best in a simulated schedule for nearly all
+// sizes up to 4096 rows, and no size longer than with the shares that make about
+// 512 blocks (2644 rows: 4 shares 34.5 tiles, 3 shares 31; 128 rows over 2048
+// positions: 16 shares). Up to 2048 blocks, which bounds the partials. Measured
+// with the order of the blocks, an attention layer of 2644 fp32 tokens 548 ->
+// 496 us; 128 tokens over 1920 as before (its share count is the same).
+int bf3_splits(int rows, int heads, int kv, int tiles) {
+    constexpr int kCus = 256;
+    const int qt = ceil_div(rows, 32), first = tiles - qt > 0 ? tiles - qt : 0;  // tiles every row sees
+    double best = 0;
+    int best_s = 1;
+    for (int s = 1; s <= kMaxShares && s <= tiles && (s == 1 || long(kv) * qt * s <= 2048); ++s) {
+        auto block = [&](int q) { return 1.5 + double(ceil_div(long(first + q + 1), s)); };
+        const long blocks = long(kv) * qt * s;
+        double t = kv * (qt * (first + 0.5 * (qt + 1)) + 1.5 * s * qt) / kCus;
+        t = t > block(qt - 1) ? t : block(qt - 1);
+        for (long j = 1; kCus * j < blocks && j < 64; ++j) {
+            const double u = double(j + 1) * block(int(qt - 1 - kCus * j / (long(kv) * s)));
+            t = t > u ? t : u;
+        }
+        if (s > 1) t += 1 + double(rows) * heads * 258 * 8 * s / 5e6 / 5.4;
+        if (s == 1 || t < best) {
+            best = t;
+            best_s = s;
+        }
+    }
+    return best_s;
+}
+// The other shapes: about 512 blocks.
+int prefill_splits(int rows, int heads, int kv, int d, int tiles) {
+    if (bf3_shape(d, heads, kv)) return bf3_splits(rows, heads, kv, tiles);
     const long blocks = long(ceil_div(rows, 32)) * (kv > 0 ? kv : 1);
     const long most = tiles < kMaxShares ? tiles : kMaxShares, s = (512 + blocks - 1) / blocks;
     return int(s < 1 ? 1 : s > most ? most : s);
@@ -998,7 +1034,7 @@ int prefill_splits(int rows, int kv, int tiles) {
 // Scratch of a prefill call, in floats: the split partials, then (head dim
 // 256, 4 query heads per KV head) the K and V^T planes at a 256-byte boundary.
 size_t prefill_parts_floats(int tokens, int heads, int kv, int d, int tiles) {
-    const int splits = prefill_splits(tokens, kv, tiles);
+    const int splits = prefill_splits(tokens, heads, kv, d, tiles);
     return splits > 1 ? (size_t(tokens) * heads * splits * (d + 2) + 63) / 64 * 64 : 0;
 }
 
@@ -1045,7 +1081,7 @@ int run_attention_read(hipStream_t s, int heads_count, const Params& p, float* s
     }
     if (prefill_path(a.d, group, a.rows)) {
         const int tiles = prefill_tiles(a.length0, a.rows);
-        a.splits = prefill_splits(a.rows, a.kv, tiles);
+        a.splits = prefill_splits(a.rows, a.heads, a.kv, a.d, tiles);
         const size_t parts = prefill_parts_floats(a.rows, a.heads, a.kv, a.d, tiles);
         if (parts > scratch_len) return int(hipErrorInvalidValue);
         if (a.splits > 1) a.parts = scratch;

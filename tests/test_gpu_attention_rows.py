@@ -40,7 +40,8 @@ def test_decode_row(both, d, heads, kv, length):
     parity(got, want, where=f"decode row {d} {heads}/{kv} {length}")
 
 
-@pytest.mark.parametrize("length,rows", [(1, 9), (1, 33), (30, 40), (500, 32), (513, 17), (1000, 65)])
+@pytest.mark.parametrize("length,rows", [(1, 9), (1, 33), (30, 40), (500, 32), (513, 17), (1000, 65),
+                                         (1, 700), (40, 1037)])  # several blocks per CU
 def test_shares(both, length, rows):
     """KV shares from one tile each up to the most, rows past a 32-row tile."""
     print(f"shares length={length} rows={rows}", flush=True)
