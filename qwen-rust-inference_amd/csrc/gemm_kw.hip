@@ -1,5 +1,5 @@
 // Projections of few to a few hundred tokens on gfx950: Y[M, N] = X[M, K]
-// W[N, K]^T to fp32 accuracy, with K split over the 8 waves of a block.
+// W[N, K]^T to fp32 accuracy, with K split over the 4 waves of a block.
 //
 // X comes as the three BF16 planes of its values in MFMA fragment order (P3,
 // common.h); W as its planes (prepared matrices) or in its own format (fp32,
