@@ -191,7 +191,7 @@ __device__ __forceinline__ void prep_task(const Params& a, int gated, int qkn, i
             // tile are 8 contiguous float4 per matrix, read before the 32 MFMAs
             // K K^T as rows t, columns s; Q K^T transposed (rows s, columns t), so that a lane's
             // four values go to four 256-byte runs of the record's L (its tiles past the diagonal
-            // are neither written nor used)
+            // are not written: the scan loads them and multiplies none, see scan_group)
             const float* pa = &ks[16 * (qk ? sj : ti) + lc][32 * q];
             const float* pb = qk ? &qs[16 * ti + lc][32 * q] : &ks[16 * sj + lc][32 * q];
             // two independent accumulator chains (k below and above 64 within each lane group's
@@ -409,7 +409,11 @@ __device__ __forceinline__ void scan_group(const Params& a, int c0, int chunks, 
     auto& dl = S.dl;
     const bool active = ALL || threadIdx.x < 256;
     const int h = i / kSlices, js = i % kSlices;
-    const int tid = threadIdx.x, w = (tid >> 6) & 3, l = tid & 63, lc = l & 15, q = l >> 4;
+    // w is a scalar, and must be: wave w multiplies only the L tiles m <= w (prep writes no
+    // others), and an MFMA ignores EXEC, so only a scalar branch keeps it from running. Under a
+    // per-lane condition the compiler masks the lanes and may run it all the same.
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6) & 3;
+    const int l = tid & 63, lc = l & 15, q = l >> 4;
     const int vh = a.n[3], tokens = a.n[4] > 0 ? a.n[4] : 1;
     float* state = a.p[4] + size_t(h) * kD * kD + js * kSlice;
     // the output as a buffer of exactly tokens x vh x kD floats (its size is
@@ -467,7 +471,7 @@ __device__ __forceinline__ void scan_group(const Params& a, int c0, int chunks, 
             for (int m = 0; m < 4; ++m) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    if (m <= w) oacc = mfma16(lv[m][e], db[m][e], oacc);  // L is zero past the tile's last token
+                    if (m <= w) oacc = mfma16(lv[m][e], db[m][e], oacc);  // (a branch: w is a scalar)
                     s0 = mfma16(k0[m][e], db[m][e], s0);
                     s1 = mfma16(k1[m][e], db[m][e], s1);
                 }

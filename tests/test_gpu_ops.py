@@ -2,13 +2,15 @@
 CPU op bridge (the restatement of the reference's op bodies) on the same
 seeded inputs, or against fp64 for the projections; argmax and the
 embedding ops bit-exact."""
+import ctypes
+
 import numpy as np
 import pytest
 
 from bridges import both, rnd
 from conftest import ROOT
 from parity import FP32_RTOL, dot_bound, parity
-from qwen_mi355x.bridge import Bridge, pack_bf16, pack_int8
+from qwen_mi355x.bridge import Bridge, Params, pack_bf16, pack_int8
 
 import oracle as O
 
@@ -728,6 +730,44 @@ def test_delta_rule_chunked(gpu, cpu, tokens, gated, a_log, heads):
                 [kd, vd, heads, heads, tokens, stride, 0])
     parity(g[0], c[0], where="core")
     parity(g[4], c[4], where="state")
+
+
+@pytest.mark.parametrize("tokens", [16, 65, 130, 64 * 66 + 3])
+def test_delta_rule_record_scratch(gpu, tokens):
+    """The chunked rule's outputs do not depend on what its record buffer holds
+    beforehand: zeros (a fresh allocation) and NaN give the same bits, over one
+    chunk, several, and past 64 chunks (the scan beside the next group's prep).
+    Prep leaves the tiles of L past the diagonal unwritten."""
+    print(f"delta_rule record scratch tokens={tokens}", flush=True)
+    heads, d = 4, 128
+    rng = np.random.default_rng(tokens)
+    q, k = _unit_rows(rng, tokens * heads, d, 1 / np.sqrt(d)), _unit_rows(rng, tokens * heads, d)
+    v, state = rnd(rng, tokens * heads * d), rnd(rng, heads * d * d, 0.5)
+    decay = (-0.05 - np.abs(rnd(rng, tokens * heads, 0.1))).astype(np.float32)
+    beta = (0.5 + rnd(rng, tokens * heads, 0.2)).clip(0, 1).astype(np.float32)
+    # the bridge's own launcher (csrc/common.h), with a record buffer of the test's
+    need = getattr(gpu.L, "_ZN2qr26delta_rule_chunked_scratchERK6Params")
+    launch = getattr(gpu.L, "_ZN2qr22run_delta_rule_chunkedEP12ihipStream_tbRK6ParamsPfmb")
+    need.restype, launch.restype = ctypes.c_size_t, ctypes.c_int
+    ins = [gpu.upload(x) for x in (q, k, v, decay, beta)]
+    got = []
+    for fill in (0.0, np.nan):
+        core, s = gpu.alloc(tokens * heads * d), gpu.upload(state)
+        a = Params()
+        for i, b in enumerate([core, ins[0], ins[1], ins[2], s, ins[3], ins[4]]):
+            a.p[i] = b.ptr
+        for i, n in enumerate([d, d, heads, heads, tokens, heads * d]):
+            a.n[i] = n
+        words = need(ctypes.byref(a))
+        scratch = gpu.upload(np.full(words, fill, np.float32))
+        gpu.sync()
+        st = launch(None, ctypes.c_bool(False), ctypes.byref(a), ctypes.c_void_p(scratch.ptr), ctypes.c_size_t(words),
+                    ctypes.c_bool(False))
+        assert st == 0
+        got.append((core.read(), s.read()))
+    for one, other in zip(*got):
+        assert np.isfinite(one).all()
+        assert np.array_equal(one, other)
 
 
 @pytest.mark.parametrize("d,rot,heads,kv,tokens,pos", [(256, 64, 8, 2, 1, 453), (256, 64, 8, 2, 3, 8190),
