@@ -214,9 +214,12 @@ const Context::Prepared* prepared_for(Context* c, qr::WeightType t, const void* 
     return batch < kPrefillMinBatch ? nullptr : planes_of(c, t, a, rows, cols);
 }
 // Matrix a as an operand of the few-token kernels (gemm_kw.hip): its planes,
-// or the matrix itself; false when they do not take it.
+// or the matrix itself; false when they do not take it. A few-row matrix that
+// gemm_ab takes joins the launch of wider matrices of its group (`joins`); on
+// its own it stays there (16 x 1024 fp32, 5 to 640 tokens: 6.1-7.1 us there,
+// 8.5-13.7 here behind a split of the input). The results are the same bits.
 bool kw_item(Context* c, qr::WeightType t, float* y, const void* a, const float* x, int rows, int cols, int batch,
-             qr::KwItem* out) {
+             bool joins, qr::KwItem* out) {
     if (batch < kPlanesMinBatch || !qr::p3_cols_ok(cols) || reinterpret_cast<uintptr_t>(x) % 16 != 0) return false;
     const float* scale = t == qr::WeightType::I8 ? static_cast<const float*>(a) : nullptr;
     if (const Context::Prepared* p = planes_of(c, t, a, rows, cols)) {
@@ -226,6 +229,7 @@ bool kw_item(Context* c, qr::WeightType t, float* y, const void* a, const float*
     } else {
         return false;
     }
+    if (qr::kw_few_rows(*out) && !joins && qr::gemm_ab_ok(t, a, x, rows, cols, batch)) return false;
     return qr::kw_wanted(t, out->raw, batch, rows);
 }
 // A planes buffer large enough for batch rows of cols (queued work on the old
@@ -345,10 +349,11 @@ int rope_table(Context* c, float theta, int rot, const float** out) {
 int project(Context* c, qr::WeightType t, float* y, const void* a, const float* x, int rows, int cols, int batch) {
     if (rows < 1 || cols < 1 || batch < 1) return fail(c, "projection shape", -1);
     qr::KwItem kw;
-    if (kw_item(c, t, y, a, x, rows, cols, batch, &kw)) {
-        if (int st = split_input(c, x, cols, batch)) return st;
+    if (kw_item(c, t, y, a, x, rows, cols, batch, false, &kw)) {
+        if (!qr::kw_few_rows(kw))
+            if (int st = split_input(c, x, cols, batch)) return st;
         auto s = scope(c, [&] { return std::string("gemm_") + wname(t) + "_kw " + shape(rows, cols, batch); });
-        return launched(c, "gemm_kw", qr::kw_gemm(c->stream, t, &kw, 1, c->xp, batch, cols));
+        return launched(c, "gemm_kw", qr::kw_gemm(c->stream, t, &kw, 1, c->xp, x, batch, cols));
     }
     if (const Context::Prepared* p = prepared_for(c, t, a, rows, cols, batch)) {
         if (int st = split_input(c, x, cols, batch)) return st;
@@ -374,19 +379,24 @@ int group(Context* c, qr::WeightType t, int n, const QrProjection* items, const 
         bool split = false;  // x's planes, made at the group's first matrix that takes them
         // the matrices of the few-token kernels, up to kKwItems to a launch
         qr::KwItem kw[qr::kKwItems], it;
-        auto few = [&](int i) { return kw_item(c, t, items[i].y, items[i].a, x, items[i].rows, cols, batch, &it); };
+        bool wide = false;  // a matrix of the few-token kernels that takes x's planes
+        auto few = [&](int i) {
+            return kw_item(c, t, items[i].y, items[i].a, x, items[i].rows, cols, batch, wide, &it);
+        };
+        for (int i = 0; i < n && !wide; ++i) wide = few(i) && !qr::kw_few_rows(it);
         for (int i = 0, m = 0; i < n; ++i) {
             if (few(i)) kw[m++] = it;
             if (m == 0 || (m < qr::kKwItems && i + 1 < n)) continue;
-            if (!split)
+            if (wide && !split) {
                 if (int st = split_input(c, x, cols, batch)) return st;
-            split = true;
+                split = true;
+            }
             auto s = scope(c, [&] {
                 std::string l = std::string("gemm_") + wname(t) + "_kw_group";
                 for (int k = 0; k < m; ++k) l += (k ? "+" : " ") + shape(kw[k].rows, cols, 1);
                 return l + " t" + std::to_string(batch);
             });
-            if (int st = launched(c, "gemm_kw", qr::kw_gemm(c->stream, t, kw, m, c->xp, batch, cols))) return st;
+            if (int st = launched(c, "gemm_kw", qr::kw_gemm(c->stream, t, kw, m, c->xp, x, batch, cols))) return st;
             m = 0;
         }
         for (int i = 0; i < n; ++i) {
@@ -441,8 +451,8 @@ int glu(Context* c, qr::WeightType t, float* product, float* gate_y, float* up_y
         // a few to a few hundred tokens: one kernel over the matrices' planes or the matrices themselves
         qr::KwItem kg, ku;
         if (rows % 32 == 0 && reinterpret_cast<uintptr_t>(product) % 16 == 0 &&
-            kw_item(c, t, product, gate, x, rows, cols, batch, &kg) &&
-            kw_item(c, t, product, up, x, rows, cols, batch, &ku) && kg.raw == ku.raw &&
+            kw_item(c, t, product, gate, x, rows, cols, batch, false, &kg) &&
+            kw_item(c, t, product, up, x, rows, cols, batch, false, &ku) && kg.raw == ku.raw &&
             qr::kw_wanted(t, kg.raw, batch, 2 * rows)) {
             if (int st = split_input(c, x, cols, batch)) return st;
             const bool planes = planes_wanted(c, rows, batch);

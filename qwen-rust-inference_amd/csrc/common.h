@@ -134,7 +134,7 @@ size_t p3_glu_scratch(int M, int rows, int K, int wplanes = 3);
 // BF16 / int8) or in its own format (raw: fp32, packed BF16, or the int8
 // values that follow the scales; kw_raw_ok), K % 32 == 0. int8: `scale` the
 // row scales, applied after the sum.
-constexpr int kKwItems = 8, kKwMaxTokens = 640;
+constexpr int kKwItems = 8, kKwMaxTokens = 640, kKwFewRows = 16;
 struct KwItem {
     float* y;
     const void* w;
@@ -142,12 +142,16 @@ struct KwItem {
     int rows;
     bool raw;
 };
+// A matrix of at most kKwFewRows rows in its own format is multiplied in whole
+// fp32 products from X itself (16-byte aligned), not from its planes.
+inline bool kw_few_rows(const KwItem& i) { return i.raw && i.rows <= kKwFewRows; }
 // Whether a projection of M tokens and so many rows (the GLU: gate's and up's
 // together) runs faster here than on the prefill GEMMs.
 bool kw_wanted(WeightType t, bool raw, int M, int rows);
 // Whether a matrix without planes has the alignment the kernels load it by.
 bool kw_raw_ok(WeightType t, const void* a, int rows, int cols);
-int kw_gemm(hipStream_t s, WeightType t, const KwItem* items, int n, const __bf16* xp, int M, int K);
+// xp may be null when every item is a few-row one.
+int kw_gemm(hipStream_t s, WeightType t, const KwItem* items, int n, const __bf16* xp, const float* x, int M, int K);
 // product = silu(X G^T) * (X U^T) and, when set, its P3 planes; rows % 32 == 0,
 // product 16-byte aligned.
 int kw_glu(hipStream_t s, WeightType t, float* product, __bf16* planes, const KwItem& gate, const KwItem& up,

@@ -52,6 +52,7 @@ constexpr int NW = 4;
 // One launch: up to kKwItems matrices of one X (their column tiles in order).
 struct KwArgs {
     const __bf16* xp;
+    const float* x;  // X itself (read for the few-row matrices only)
     int M, kt, tiles_m, tiles_n, count;  // kt: K / 16
     struct Item {
         float* y;
@@ -289,6 +290,66 @@ __device__ __forceinline__ void store4(const KwArgs::Item& it, int m, int n, f4v
     }
 }
 
+// 16 tokens of a matrix of at most 16 rows in its own format (the DeltaNet a
+// and b, whose outputs set the decay and beta of every token) as whole fp32
+// products on v_mfma_f32_16x16x4_f32, X from its fp32 values: the arithmetic of
+// gemm_ab_mfma_kernel (gemm.hip) to the bit, so that such a matrix gives the
+// same result alone and in a group, and an infinite or very large value stays
+// what it is (split into BF16 parts it becomes NaN). Step m is 16 columns, MFMA
+// e of it takes k = 16 m + 4 (lane / 16) + e; the even steps of wave w are those
+// of wave w there, the odd ones those of wave w + 4, and the eight partial tiles
+// are added in that order. A block takes 16 tokens whatever the launch's tile
+// (kFewTokens; up to four blocks stand in the place of one tile): with all of a
+// 64-token tile in one block these blocks ended last (DeltaNet layer, 77 BF16
+// tokens: 65.8 us, now 59.3 as with split products; 128 fp32 tokens: 75.6, now
+// 70.4, with split products 72.3).
+constexpr int kFewTokens = 16;
+template <WeightType T>
+__device__ __forceinline__ void few_rows(const KwArgs& p, const KwArgs::Item& it, int m0, float* part) {
+    constexpr int B = 16;  // steps in flight (K = 1024: all of a wave's)
+    const int lane = int(threadIdx.x) & 63, w = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+    const int lr = lane & 15, g = lane >> 4, K = 16 * p.kt;
+    const size_t wr = size_t(min(lr, it.rows - 1)) * K;  // (rows past the matrix or the tokens: not stored)
+    const float* const xr = p.x + size_t(min(m0 + lr, p.M - 1)) * K;
+    f4v acc[2] = {f4v{0.f, 0.f, 0.f, 0.f}, f4v{0.f, 0.f, 0.f, 0.f}};
+    for (int mb = w; mb < p.kt; mb += NW * B) {
+        f4v wv[B], xv[B];
+#pragma unroll
+        for (int j = 0; j < B; ++j) {
+            const int k = 16 * min(mb + NW * j, p.kt - 1) + 4 * g;
+            xv[j] = *reinterpret_cast<const f4v*>(xr + k);
+            if constexpr (T == WeightType::F32) {
+                wv[j] = *reinterpret_cast<const f4v*>(static_cast<const float*>(it.w) + wr + k);
+            } else if constexpr (T == WeightType::BF16) {
+                const uint2 v = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(it.w) + wr + k);
+                wv[j] = f4v{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
+                            __uint_as_float(v.y & 0xffff0000u)};
+            } else {
+                const unsigned v = *reinterpret_cast<const unsigned*>(static_cast<const int8_t*>(it.w) + wr + k);
+                wv[j] = f4v{float(int(v << 24) >> 24), float(int(v << 16) >> 24), float(int(v << 8) >> 24),
+                            float(int(v) >> 24)};
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < B; ++j)
+            if (mb + NW * j < p.kt)  // (a scalar)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    acc[j & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[j][e], wv[j][e], acc[j & 1], 0, 0, 0);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) part[((w + NW * h) * kFewTokens + 4 * g + r) * 16 + lr] = acc[h][r];
+    __syncthreads();
+    const int m = int(threadIdx.x) / 16, n = int(threadIdx.x) % 16;
+    if (m0 + m >= p.M || n >= it.rows) return;
+    float s = part[threadIdx.x];
+#pragma unroll
+    for (int v = 1; v < 2 * NW; ++v) s += part[v * kFewTokens * 16 + threadIdx.x];
+    it.y[size_t(m0 + m) * it.rows + n] = it.scale ? it.scale[n] * s : s;
+}
+
 // Two waves per SIMD (256 registers each) also keep the accumulators out of the
 // AGPRs: with 512 registers to a wave the compiler moved them there and back at
 // every branch of the ring's end and read the last one before its MFMA had
@@ -306,13 +367,19 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     const KwArgs::Item& it = p.it[item];
     const int m0 = mt * TM, n0 = GLU ? 32 * nt : TN * (nt - it.first);
     const int kt = p.kt;
+    if constexpr (!GLU)
+        if (it.raw && it.rows <= kKwFewRows) {
+            const int t0 = m0 + kFewTokens * (nt - it.first);
+            if (t0 < p.M) few_rows<T>(p, it, t0, part);
+            return;
+        }
     const char* xb[TMT];
 #pragma unroll
     for (int i = 0; i < TMT; ++i)
         xb[i] = reinterpret_cast<const char*>(p.xp) + size_t(mt * TMT + i) * kt * 3072 + 16 * lane;
     f16v acc[TMT][TNT];
     const char* wb[TNT];
-    if (!GLU && TNT == 2 && it.raw && it.rows <= 32) {  // a few-row matrix (the DeltaNet a and b): half the tile
+    if (!GLU && TNT == 2 && it.raw && it.rows <= 32) {  // half the tile
         const char* wb1[1] = {reinterpret_cast<const char*>(it.w) +
                               (size_t(min(lane & 31, it.rows - 1)) * kt * 16 + 8 * (lane >> 5)) * kRawBytes<T>};
         f16v half[TMT][1];
@@ -510,9 +577,10 @@ long blocks_of(const KwItem* items, int n, int M, Tile t) {
 // weights in their own format are split in the kernel, once per 32 x 16
 // operand: 64 x 32 splits half as many as 32 x 64 (down, 300 tokens: 28.8
 // against 34.5 us). The 32 x 16 tile is for matrices of a width worth
-// spreading (a 16-row matrix keeps the arithmetic of the wider tiles, whose
-// sums are bitwise the same for every tile but this one, so that it gives the
-// same result alone and in a group).
+// spreading (few_rows runs in the wider ones). Every other tile forms the same
+// sums to the bit; in this one a K step is twice as deep and they round
+// differently, so a matrix of 128 rows or more may differ in its last bits
+// between a call of its own and a group that makes more than 256 such tiles.
 Tile pick_tile(WeightType t, const KwItem* items, int n, int M) {
     bool narrow = true;
     for (int i = 0; i < n; ++i) narrow = narrow && items[i].rows >= 128;
@@ -539,20 +607,23 @@ bool kw_raw_ok(WeightType t, const void* a, int rows, int cols) {
     return p3_cols_ok(cols) && reinterpret_cast<uintptr_t>(a) % 16 == 0 && (t != WeightType::I8 || rows % 2 == 0);
 }
 
-int kw_gemm(hipStream_t s, WeightType t, const KwItem* items, int n, const __bf16* xp, int M, int K) {
-    if (M < 1 || n < 1 || n > kKwItems || !p3_cols_ok(K)) return int(hipErrorInvalidValue);
+int kw_gemm(hipStream_t s, WeightType t, const KwItem* items, int n, const __bf16* xp, const float* x, int M, int K) {
+    if (M < 1 || n < 1 || n > kKwItems || !p3_cols_ok(K) || reinterpret_cast<uintptr_t>(x) % 16)
+        return int(hipErrorInvalidValue);
     for (int i = 0; i < n; ++i)
-        if (items[i].rows < 1 || reinterpret_cast<uintptr_t>(items[i].scale) % 16) return int(hipErrorInvalidValue);
+        if (items[i].rows < 1 || reinterpret_cast<uintptr_t>(items[i].scale) % 16 || !(kw_few_rows(items[i]) ? x != nullptr : xp != nullptr))
+            return int(hipErrorInvalidValue);
     const Tile tile = pick_tile(t, items, n, M);
     KwArgs a{};
     a.xp = xp;
+    a.x = x;
     a.M = M;
     a.kt = K / 16;
     a.tiles_m = int(ceil_div(M, tile_m(tile)));
     a.count = n;
     for (int i = 0; i < n; ++i) {
         a.it[i] = KwArgs::Item{items[i].y, items[i].w, items[i].scale, items[i].rows, a.tiles_n, items[i].raw ? 1 : 0};
-        a.tiles_n += int(ceil_div(items[i].rows, tile_n(tile)));
+        a.tiles_n += kw_few_rows(items[i]) ? tile_m(tile) / kFewTokens : int(ceil_div(items[i].rows, tile_n(tile)));
     }
     return launch_t(s, t, tile, false, a);
 }

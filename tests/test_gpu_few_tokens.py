@@ -138,3 +138,56 @@ def test_operands_off_alignment(gpu, kind):
         gpu.gemm(o, m, v, rows, cols, batch, kind=kind)
         got = y.read()[1:] if isinstance(o, At) else y.read(batch * rows)
         near(got.reshape(batch, rows), X, W, scale)
+
+
+@pytest.mark.parametrize("kind", ["f32", "bf16", "i8"])
+@pytest.mark.parametrize("prepared", [True, False])
+@pytest.mark.parametrize("rows,cols,batch", [(16, 1024, 5), (16, 1024, 128), (16, 1024, 640), (16, 96, 33), (10, 32, 23),
+                                             (1, 160, 64), (7, 1024, 31), (16, 2048, 77)])
+def test_few_rows(gpu, kind, prepared, rows, cols, batch):
+    """A matrix of at most 16 rows (the DeltaNet a and b): whole fp32 products,
+    the same bits alone and beside wider matrices (200 rows: the narrow tiles'
+    sizes; 5120: the widest), the wider ones unchanged by its company."""
+    print(f"few rows {kind} {rows}x{cols} batch {batch} prepared {prepared}", flush=True)
+    rng = np.random.default_rng(rows + cols + batch)
+    x = rng.standard_normal(batch * cols).astype(np.float32)
+    X, xb = x.reshape(batch, cols).astype(np.float64), gpu.upload(x)
+    mats = {r: matrix(kind, (rng.standard_normal(r * cols) * 0.02).astype(np.float32), r, cols)
+            for r in (rows, 200, 5120)}
+    bufs = {r: gpu.upload(m[0]) for r, m in mats.items()}
+    if prepared:
+        for r in (200, 5120):
+            gpu.prepare(bufs[r], r, cols, kind=kind)
+    alone = gpu.alloc(batch * rows)
+    gpu.gemm(alone, bufs[rows], xb, rows, cols, batch, kind=kind)
+    near(alone.read().reshape(batch, rows), X, *mats[rows][1:])
+    for wide in (200, 5120):
+        ys = [gpu.alloc(batch * r) for r in (wide, rows, rows)]
+        gpu.group([(ys[0], bufs[wide], wide), (ys[1], bufs[rows], rows), (ys[2], bufs[rows], rows)], xb, cols, batch,
+                  kind=kind)
+        near(ys[0].read().reshape(batch, wide), X, *mats[wide][1:])
+        for y in ys[1:]:
+            assert np.array_equal(y.read(), alone.read()), wide
+
+
+@pytest.mark.parametrize("kind", ["f32", "bf16", "i8"])
+def test_few_rows_keep_infinities(gpu, kind):
+    """Beside wider matrices the few-row ones keep an infinite input infinite
+    and the largest fp32 values finite (their BF16 parts are not)."""
+    rows, cols, batch = 16, 1024, 40
+    rng = np.random.default_rng(5)
+    words, W, scale = matrix(kind, (0.01 + rng.random(rows * cols) * 0.02).astype(np.float32), rows, cols)
+    wide = matrix(kind, (rng.standard_normal(512 * cols) * 0.02).astype(np.float32), 512, cols)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    x[3, 700] = np.inf
+    x[17, 5] = -np.inf
+    x[33, 9] = np.finfo(np.float32).max
+    if kind == "i8":
+        x[33, 9] /= 256  # (the integers' products are scaled after the sum)
+    ys = [gpu.alloc(batch * r) for r in (512, rows)]
+    gpu.group([(ys[0], gpu.upload(wide[0]), 512), (ys[1], gpu.upload(words), rows)], gpu.upload(x.reshape(-1)), cols,
+              batch, kind=kind)
+    got = ys[1].read().reshape(batch, rows)
+    assert np.all(got[3] == np.inf) and np.all(got[17] == -np.inf)
+    rest = [t for t in range(batch) if t not in (3, 17)]
+    near(got[rest], x[rest].astype(np.float64), W, scale)
