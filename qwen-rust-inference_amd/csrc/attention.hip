@@ -253,6 +253,10 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(ReadArgs a) {
             if (lane == 0) corr[b][g] = c;
         }
         __syncthreads();
+        if (c0 + CH > end)  // values of positions past the span stand for none (not 0 * inf)
+#pragma unroll
+            for (int s = 0; s < VS; ++s)
+                if (c0 + CPW * wave + VP * s + vslot >= end) vx[s] = f4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int g = 0; g < G; ++g) acc[g] *= corr[b][g];
 #pragma unroll

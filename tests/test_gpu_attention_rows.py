@@ -62,3 +62,21 @@ def test_large_scores(both):
                 rnd(rng, heads * d)]
         got, want = (read(b, d, heads, kv, length, 1, data) for b in both)
         parity(got, want, where=f"scale {scale}")
+
+
+@pytest.mark.parametrize("heads,kv,length,rows", [(8, 2, 33, 1), (8, 2, 17, 1), (8, 1, 1, 9), (8, 1, 33, 9)])
+def test_infinite_values(both, heads, kv, length, rows):
+    """An infinite value at a span's first position reaches its own dim of the
+    context and no other, also where the span ends inside a chunk."""
+    d = 256
+    rng = np.random.default_rng(length + rows)
+    n = length + rows
+    values = rnd(rng, n * kv * d).reshape(n, kv, d)
+    at = (length - 1) // 16 * 16 if rows == 1 else 0
+    values[at, :, 3] = np.inf
+    values[at, :, 250] = -np.inf
+    data = [rnd(rng, rows * heads * d), rnd(rng, n * kv * d), values.reshape(-1), rnd(rng, rows * heads * d)]
+    got, want = (read(b, d, heads, kv, length, rows, data).reshape(rows, heads, d) for b in both)
+    assert np.all(got[..., 3] == np.inf) and np.all(got[..., 250] == -np.inf)
+    rest = [i for i in range(d) if i not in (3, 250)]
+    parity(got[..., rest], want[..., rest], where=f"inf {length} {rows}")
