@@ -80,3 +80,23 @@ def test_infinite_values(both, heads, kv, length, rows):
     assert np.all(got[..., 3] == np.inf) and np.all(got[..., 250] == -np.inf)
     rest = [i for i in range(d) if i not in (3, 250)]
     parity(got[..., rest], want[..., rest], where=f"inf {length} {rows}")
+
+
+@pytest.mark.parametrize("heads,kv,rows", [(8, 1, 12), (16, 2, 9)])
+def test_long_rows_sum_in_chunks(both, heads, kv, rows):
+    """Equal scores (q = 0) over 1920 positions of values in (0, 1): the context
+    is the values' mean, its error that of the sum alone. One chain of 480
+    additions per wave is off by about 2^-24 sqrt(480) / 3 / 2 = 2.2e-7 (2-norm;
+    partial sums grow evenly, four waves' errors average; measured 1.5e-7), chunks
+    of 8 with 60 additions between them by 8e-8 (6.5e-8), the division's 3e-8 included."""
+    d, length = 256, 1920
+    rng = np.random.default_rng(7)
+    n = length + rows
+    values = rng.random((n, kv, d)).astype(np.float32)
+    data = [np.zeros(rows * heads * d, np.float32), rnd(rng, n * kv * d), values.reshape(-1),
+            np.full(rows * heads * d, 40.0, np.float32)]  # sigmoid(40) rounds to 1
+    got = read(both[0], d, heads, kv, length, rows, data).reshape(rows, kv, heads // kv, d).astype(np.float64)
+    want = np.stack([values[:length + r].astype(np.float64).mean(0) for r in range(rows)])[:, :, None]
+    err = np.sqrt(np.sum((got - want) ** 2) / np.sum(np.broadcast_to(want, got.shape) ** 2))
+    print(f"error {err:.3e}", flush=True)
+    assert err < 1.1e-7, err
