@@ -245,8 +245,10 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(ReadArgs a) {
             const int g = wave + 4 * h;
             if (g >= G) break;
             const float x = lane < CH ? ss[b][lane][g] : -INFINITY;
-            const float mn = fmaxf(m[h], wave_max(x));  // finite: the chunk's first position is live
-            const float c = expf(m[h] - mn), w = expf(x - mn);
+            // -inf scores (and lanes past the span) weigh nothing, a maximum of -inf scales nothing;
+            // a span of nothing else leaves (-inf, 0, 0), which the merge skips
+            const float mn = fmaxf(m[h], wave_max(x));
+            const float c = m[h] == -INFINITY ? 0.f : expf(m[h] - mn), w = x == -INFINITY ? 0.f : expf(x - mn);
             l[h] = l[h] * c + wave_sum(w);
             m[h] = mn;
             if (lane < CH) ss[b][lane][g] = w;

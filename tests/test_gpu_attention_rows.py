@@ -100,3 +100,22 @@ def test_long_rows_sum_in_chunks(both, heads, kv, rows):
     err = np.sqrt(np.sum((got - want) ** 2) / np.sum(np.broadcast_to(want, got.shape) ** 2))
     print(f"error {err:.3e}", flush=True)
     assert err < 1.1e-7, err
+
+
+@pytest.mark.parametrize("d,heads,kv", [(256, 8, 2), (256, 8, 1), (128, 3, 3), (64, 4, 2)])
+@pytest.mark.parametrize("length,dead", [(300, 200), (300, 31), (64, 40), (4111, 4100)])
+def test_scores_of_minus_infinity(both, d, heads, kv, length, dead):
+    """The first `dead` positions score -inf (whole chunks, spans and merge
+    inputs among them): they weigh nothing. All of them: NaN, as the CPU op."""
+    rng = np.random.default_rng(d + length + dead)
+    q = rnd(rng, heads * d).reshape(heads, d)
+    q[:, 0] = np.abs(q[:, 0]) + 0.1
+    keys = rnd(rng, length * kv * d).reshape(length, kv, d)
+    keys[:dead, :, 0] = -np.inf
+    data = [q.reshape(-1), keys.reshape(-1), rnd(rng, length * kv * d), rnd(rng, heads * d)]
+    got, want = (read(b, d, heads, kv, length, 1, data) for b in both)
+    parity(got, want, where=f"-inf {d} {length} {dead}")
+    keys[:, :, 0] = -np.inf
+    data[1] = keys.reshape(-1)
+    for b in both:
+        assert np.isnan(read(b, d, heads, kv, length, 1, data)).all()
