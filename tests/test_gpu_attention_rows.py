@@ -119,3 +119,16 @@ def test_scores_of_minus_infinity(both, d, heads, kv, length, dead):
     data[1] = keys.reshape(-1)
     for b in both:
         assert np.isnan(read(b, d, heads, kv, length, 1, data)).all()
+
+
+@pytest.mark.parametrize("length,rows", [(1, 9), (77, 40), (500, 33)])
+def test_rows_of_eight_heads(both, length, rows):
+    """Head dim 256 with eight query heads per KV head has no tiled prefill
+    form: each row of a chunk is one block over its whole length."""
+    print(f"rows of 8 heads length={length} rows={rows}", flush=True)
+    d, heads, kv = 256, 8, 1
+    rng = np.random.default_rng(length + rows)
+    n = length + rows
+    data = [rnd(rng, rows * heads * d), rnd(rng, n * kv * d), rnd(rng, n * kv * d), rnd(rng, rows * heads * d)]
+    got, want = (read(b, d, heads, kv, length, rows, data) for b in both)
+    parity(got, want, where=f"eight heads {length} {rows}")
