@@ -350,10 +350,10 @@ __device__ __forceinline__ void few_rows(const KwArgs& p, const KwArgs::Item& it
     it.y[size_t(m0 + m) * it.rows + n] = it.scale ? it.scale[n] * s : s;
 }
 
-// Two waves per SIMD (256 registers each) also keep the accumulators out of the
-// AGPRs: with 512 registers to a wave the compiler moved them there and back at
-// every branch of the ring's end and read the last one before its MFMA had
-// written it.
+// Two waves per SIMD (256 registers each, here and in kw_narrow_kernel) also keep
+// the accumulators out of the AGPRs: with 512 registers to a wave the compiler
+// moved them there and back at every branch of the ring's end, and one build of
+// this kernel gave wrong last sums, as if read before their MFMA had written them.
 // GLU = false: a (32 TMT) x (32 TNT) tile of one item. GLU = true (TNT = 2):
 // 32 gate rows and the same 32 up rows, product = silu(g) * u and its planes.
 template <WeightType T, int TMT, int TNT, bool GLU>
@@ -452,7 +452,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
 // (32 s + 8 (l / 16)) of row l % 16 of each operand; register r of its
 // accumulator is row 4 (l / 16) + r, column l % 16.
 template <WeightType T>
-__global__ __launch_bounds__(64 * NW) void kw_narrow_kernel(KwArgs p) {
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) void kw_narrow_kernel(KwArgs p) {
     constexpr int TM = 32, TN = 16, PITCH = TN + 4, SLOT = TM * PITCH;
     constexpr int WP = kPlanes<T>;
     __shared__ __attribute__((aligned(16))) float part[NW * SLOT];
