@@ -4,7 +4,6 @@
 // and the reference entry point each one replaces: include/qwen_bridge.h.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -74,9 +73,6 @@ struct Context {
     const float* xp_src = nullptr;
     int xp_rows = 0, xp_cols = 0;
     unsigned long serial = 0, xp_serial = 0;
-    // Widths of inputs that a projection split itself (split_input), the
-    // first 16 of them.
-    int plane_widths[16] = {}, plane_width_count = 0;
     // The width of the projection that took the last RmsNormGate output right
     // after it (its rows span several groups), by group size: from then on such
     // a norm writes its planes in rows of that width.
@@ -252,10 +248,6 @@ int grow_xp(Context* c, int cols, int batch) {
     if (qr::p3_elements(batch, cols) > c->xp_len) c->xp_src = nullptr;
     return grow_planes(c, &c->xp, &c->xp_len, cols, batch);
 }
-bool split_width(const Context* c, int cols) {
-    const int* end = c->plane_widths + c->plane_width_count;
-    return std::find(c->plane_widths, end, cols) != end;
-}
 // x's P3 planes into c->xp: already there when the previous bridge call
 // produced x with them, else split now.
 int split_input(Context* c, const float* x, int cols, int batch) {
@@ -263,19 +255,16 @@ int split_input(Context* c, const float* x, int cols, int batch) {
         c->gate_width[c->gate_d] = cols;  // a gated norm's output projected: its row width
     if (c->xp_src == x && c->xp_rows == batch && c->xp_cols == cols && c->xp_serial + 1 == c->serial) return 0;
     c->xp_src = nullptr;
-    if (!split_width(c, cols) && c->plane_width_count < 16)  // from now on this width's producers write the planes
-        c->plane_widths[c->plane_width_count++] = cols;
     if (int st = grow_xp(c, cols, batch)) return st;
     auto s = scope(c, [&] { return std::string("p3_split ") + shape(batch, cols, 1); });
     return launched(c, "p3_split", qr::p3_split(c->stream, c->xp, x, batch, cols));
 }
 // Whether a producer of `rows` rows of width `cols` should also write the
-// planes: enough rows for the planes path, and a prepared matrix of that width
-// or (while the few-token kernels take matrices without planes) a projection
-// that split such an input before.
+// planes: enough rows for the planes path, and a prepared matrix of that width.
+// (Not for matrices in their own format: an engine that prepared nothing may
+// rewrite an input by other means than the bridge between two calls.)
 bool planes_wanted(Context* c, int cols, int rows) {
     if (rows < kPlanesMinBatch || !qr::p3_cols_ok(cols)) return false;
-    if (rows <= qr::kKwMaxTokens && split_width(c, cols)) return true;
     for (auto& kv : c->prepared)
         if (kv.second.cols == cols && kv.second.rows > 16) return true;
     return false;

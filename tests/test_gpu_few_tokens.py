@@ -3,6 +3,8 @@ through the C ABI against float64, at the edges of their tiles and of the rule
 that picks them: every output tile, ragged tokens and rows, K shorter than the
 block's waves, prepared matrices and matrices in their own format, groups
 longer than a launch, and operands whose alignment the kernels do not take."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -191,3 +193,36 @@ def test_few_rows_keep_infinities(gpu, kind):
     assert np.all(got[3] == np.inf) and np.all(got[17] == -np.inf)
     rest = [t for t in range(batch) if t not in (3, 17)]
     near(got[rest], x[rest].astype(np.float64), W, scale)
+
+
+@pytest.mark.parametrize("batch", [23, 128])
+def test_unprepared_inputs_may_be_rewritten(gpu, batch):
+    """Where no matrix is prepared, a projection takes its input as it lies in
+    memory: also what another context wrote there after the norm or the GLU
+    that produced it, with no call of this context in between."""
+    cols, rows = 1024, 256
+    rng = np.random.default_rng(batch)
+    b = Bridge()
+    other = Bridge()
+    try:
+        words, W, scale = matrix("i8", (rng.standard_normal(rows * cols) * 0.02).astype(np.float32), rows, cols)
+        square, _, _ = matrix("i8", (rng.standard_normal(cols * cols) * 0.02).astype(np.float32), cols, cols)
+        a, sq = b.upload(words), b.upload(square)
+        x, norm = b.upload(rng.standard_normal(batch * cols).astype(np.float32)), b.upload(np.zeros(cols, np.float32))
+        normed, gy, uy, y = b.alloc(batch * cols), b.alloc(batch * cols), b.alloc(batch * cols), b.alloc(batch * rows)
+        producers = [lambda: b.run("RMS_NORM", batch, [normed, x, norm], [cols], [1e-6, 1.0]),
+                     lambda: b.glu(normed, gy, uy, sq, sq, x, cols, cols, batch, kind="i8")]
+        for produce in producers:
+            for _ in range(2):
+                produce()
+                b.gemm(y, a, normed, rows, cols, batch, kind="i8")
+            new = rng.standard_normal(batch * cols).astype(np.float32)
+            produce()
+            assert b.L.hipDeviceSynchronize() == 0
+            assert other.L.qr_write(other.ctx, ctypes.c_void_p(normed.ptr), new.ctypes.data_as(ctypes.c_void_p),
+                                    ctypes.c_size_t(new.size)) == 0
+            b.gemm(y, a, normed, rows, cols, batch, kind="i8")
+            near(y.read().reshape(batch, rows), new.reshape(batch, cols).astype(np.float64), W, scale)
+    finally:
+        b.close()
+        other.close()
