@@ -742,7 +742,8 @@ def test_delta_rule_record_scratch(gpu, tokens):
     heads, d = 4, 128
     rng = np.random.default_rng(tokens)
     q, k = _unit_rows(rng, tokens * heads, d, 1 / np.sqrt(d)), _unit_rows(rng, tokens * heads, d)
-    v, state = rnd(rng, tokens * heads * d), rnd(rng, heads * d * d, 0.5)
+    stride = 3 * heads * d  # a token's q, k and V; the rule reads V from its third part
+    v, state = rnd(rng, tokens * stride), rnd(rng, heads * d * d, 0.5)
     decay = (-0.05 - np.abs(rnd(rng, tokens * heads, 0.1))).astype(np.float32)
     beta = (0.5 + rnd(rng, tokens * heads, 0.2)).clip(0, 1).astype(np.float32)
     # the bridge's own launcher (csrc/common.h), with a record buffer of the test's
@@ -756,7 +757,7 @@ def test_delta_rule_record_scratch(gpu, tokens):
         a = Params()
         for i, b in enumerate([core, ins[0], ins[1], ins[2], s, ins[3], ins[4]]):
             a.p[i] = b.ptr
-        for i, n in enumerate([d, d, heads, heads, tokens, heads * d]):
+        for i, n in enumerate([d, d, heads, heads, tokens, stride]):
             a.n[i] = n
         words = need(ctypes.byref(a))
         scratch = gpu.upload(np.full(words, fill, np.float32))
