@@ -639,14 +639,30 @@ def test_embed_rows(gpu, width, n):
                                              (4, 21, 2)])
 def test_conv_silu(gpu, cpu, k, tokens, snaps):
     """ConvSilu: one thread per channel walking the tokens (<= 4 tokens), the
-    16-token window kernel over prefill chunks (6146 channels: a ragged last
-    block), snapshots of the history per token."""
+    window kernel of 4 tokens per thread (kernel size 4; the 16-token one and
+    its edges: test_conv_silu_windows), one thread per token (other sizes), a
+    ragged last block (6146 channels), snapshots of the history per token."""
     rng = np.random.default_rng(k * 10 + tokens)
     ch = (6146 if tokens == 21 else 6144) if k == 4 else 24
     x, w, h = rnd(rng, tokens * ch), rnd(rng, ch * k, 0.5), rnd(rng, ch * max(k - 1, 1) * (1 + snaps))
     g, c = both(gpu, cpu, "CONV_SILU", ch, {1: x, 2: w, 3: h}, {0: tokens * ch, 3: h.size}, [k, tokens, ch, snaps])
     parity(g[0], c[0], where="conv out")
     parity(g[3], c[3], where="conv history")
+
+
+@pytest.mark.parametrize("tokens,snaps", [(5, 4), (8, 0), (255, 0), (256, 3), (257, 0), (258, 17), (272, 0), (273, 0),
+                                          (700, 0)])
+def test_conv_silu_windows(gpu, cpu, tokens, snaps):
+    """Kernel size 4 over 4 tokens per thread (up to 256) and 16 (beyond), at
+    the windows' edges: the outputs, the snapshots, and the history, whose
+    values are the last three inputs themselves."""
+    rng = np.random.default_rng(tokens)
+    k, ch = 4, 514
+    x, w, h = rnd(rng, tokens * ch), rnd(rng, ch * k, 0.5), rnd(rng, ch * (k - 1) * (1 + snaps))
+    g, c = both(gpu, cpu, "CONV_SILU", ch, {1: x, 2: w, 3: h}, {0: tokens * ch, 3: h.size}, [k, tokens, ch, snaps])
+    parity(g[0], c[0], where="conv out")
+    assert np.array_equal(g[3], c[3])
+    assert np.array_equal(g[3][:ch * (k - 1)].reshape(ch, k - 1), x.reshape(tokens, ch)[-(k - 1):].T)
 
 
 @pytest.mark.parametrize("kh,vh,d,tokens", [(16, 16, 128, 1), (16, 16, 128, 3), (2, 4, 3, 1), (4, 4, 16, 2),
