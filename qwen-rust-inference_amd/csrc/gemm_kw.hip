@@ -151,8 +151,7 @@ struct Products<WeightType::F32> {
 };
 
 // n steps through a ring of NS (even) register buffers. step(buffer, step % 2,
-// next) multiplies a buffer and, for next >= 0, loads step `next` into it plane
-// by plane as the products are done with it: loads issued in a burst after the
+// next) multiplies a buffer and, for next >= 0, loads step `next` into it plane by plane as the products are done with it: loads issued in a burst after the
 // products stall the wave (the CU's vector memory path takes 16 clocks per KiB
 // and a wave issues in order), among them they do not: q|k|v of 128 fp32 tokens
 // 14.5 -> 12.0 us, of 300 25.8 -> 20.7, the BF16 GLU of 128 tokens 11.4 -> 10.3. The main loop's
@@ -180,10 +179,13 @@ __device__ __forceinline__ void ring(int n, L&& load, S&& step) {
 }
 
 // Wave w's k tiles (w, w + NW, ...) of a (32 TMT) x (32 TNT) tile into acc. xb
-// / wb: this lane's address of each 32-row tile's k tile 0. Even and odd steps
-// sum in accumulators of their own: the chain of fp32 additions behind a sum is
-// K / 128 k tiles long, as with eight waves (error against 64 bits, DeltaNet
-// layer of 128 fp32 tokens: 6.6e-7 with one chain).
+// / wb: this lane's address of each 32-row tile's k tile 0. The leading products
+// x0 w0 sum in accumulators of their own, the others, 2^-8 of them and less, in
+// `rest`: a sum rounds once per k tile where it counts, not once per product.
+// Error against 64 bits, all products of even and all of odd steps in one
+// accumulator each -> now: k of 8 fp32 tokens 1.9e-7 -> 1.3e-7 (1.55e-7 with K
+// split over the blocks of gemm_bf3_kernel), MLP of 20 fp32 tokens 4.3e-7 ->
+// 2.7e-7, of 150 int8 tokens 3.0e-7 -> 2.1e-7; the same time.
 template <WeightType T, bool RAW, int TMT, int TNT>
 __device__ __forceinline__ void k_wave(f16v (&acc)[TMT][TNT], const char* const (&xb)[TMT], const char* const (&wb)[TNT],
                                        int kt, int w) {
@@ -204,14 +206,14 @@ __device__ __forceinline__ void k_wave(f16v (&acc)[TMT][TNT], const char* const 
 #pragma unroll
             for (int q = 0; q < 3; ++q) b.x[i][q] = *reinterpret_cast<const bf16x8*>(xb[i] + k * XSTEP + 1024 * q);
     };
-    f16v odd[TMT][TNT];
+    f16v rest[TMT][TNT];
 #pragma unroll
     for (int i = 0; i < TMT; ++i)
 #pragma unroll
         for (int j = 0; j < TNT; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = odd[i][j][r] = 0.f;
-    auto step = [&](Buf& b, int parity, int next) {
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = rest[i][j][r] = 0.f;
+    auto step = [&](Buf& b, int, int next) {
         using Pr = Products<T>;
         const size_t k = size_t(w + NW * next);
         bf16x8 h[TNT][kPlanes<T>];
@@ -229,7 +231,7 @@ __device__ __forceinline__ void k_wave(f16v (&acc)[TMT][TNT], const char* const 
             for (int i = 0; i < TMT; ++i)
 #pragma unroll
                 for (int j = 0; j < TNT; ++j) {
-                    f16v& a = parity ? odd[i][j] : acc[i][j];
+                    f16v& a = q + 1 < Pr::N ? rest[i][j] : acc[i][j];
                     a = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b.x[i][Pr::P(q)], h[j][Pr::Q(q)], a, 0, 0, 0);
                 }
             if (next < 0) continue;
@@ -250,7 +252,7 @@ __device__ __forceinline__ void k_wave(f16v (&acc)[TMT][TNT], const char* const 
 #pragma unroll
     for (int i = 0; i < TMT; ++i)
 #pragma unroll
-        for (int j = 0; j < TNT; ++j) acc[i][j] += odd[i][j];
+        for (int j = 0; j < TNT; ++j) acc[i][j] += rest[i][j];
 }
 
 // Block b's tile: the 8 XCDs take blocks in turn; XCD x takes column tiles x,
@@ -464,11 +466,13 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     // fragment lane of row r16 (of 16) and this lane's k: r16 + 32 ((l / 16) % 2), k tile l / 32 of the step
     const int fl = (lane & 15) + 32 * ((lane >> 4) & 1), fk = lane >> 5;
     const char* xb = reinterpret_cast<const char*>(p.xp) + (size_t(mt) * kt + fk) * 3072 + 16 * fl;
-    f4v acc[2][2];  // [row half][even, odd steps]
+    // [row half][the leading product of even and of odd steps, the other products]: as in k_wave, and
+    // the leading chain half as long (this tile takes the matrices of the longest K)
+    f4v acc[2][3];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc[i][0][r] = acc[i][1][r] = 0.f;
+        for (int r = 0; r < 4; ++r) acc[i][0][r] = acc[i][1][r] = acc[i][2][r] = 0.f;
     auto run = [&](auto raw, const char* wb) {
         constexpr bool RAW = decltype(raw)::value;
         constexpr int WSTEP = RAW ? 32 * kRawBytes<T> : 2 * WP * 1024;
@@ -498,9 +502,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
 #pragma unroll
             for (int q = 0; q < Pr::N; ++q) {
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
-                    acc[i][parity] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b.x[i][Pr::P(q)], h[Pr::Q(q)],
-                                                                            acc[i][parity], 0, 0, 0);
+                for (int i = 0; i < 2; ++i) {
+                    f4v& a = acc[i][q + 1 < Pr::N ? 2 : parity];
+                    a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b.x[i][Pr::P(q)], h[Pr::Q(q)], a, 0, 0, 0);
+                }
                 if (next < 0) continue;
                 __builtin_amdgcn_sched_barrier(0);
                 if (Pr::xdead(q) >= 0)
@@ -526,7 +531,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-            part[w * SLOT + (16 * i + 4 * (lane >> 4) + r) * PITCH + (lane & 15)] = acc[i][0][r] + acc[i][1][r];
+            part[w * SLOT + (16 * i + 4 * (lane >> 4) + r) * PITCH + (lane & 15)] =
+                acc[i][0][r] + (acc[i][1][r] + acc[i][2][r]);
     __syncthreads();
     if (tid < TM * TN / 4) {
         const int m = tid / (TN / 4), c = tid % (TN / 4) * 4;
