@@ -325,10 +325,12 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(ReadArgs a) {
 // (one from W = 4 on). Four dims to a lane, d / 4 lanes (up to 64) to a split's
 // partial: a wave reads whole partials, four steps' loads together, keeps (max,
 // sum, weighted sums) of its own splits, and the lanes of the same dims and the
-// waves are merged by the log-sum-exp rule, in a fixed order. A prefill chunk
-// has rows enough for one wave each; a decode row (8 heads) takes as many waves
-// as give each about four partials. At 8192 positions 6.5 us (13.4 with 16 lanes
-// per 4 dims walking 16 of 256 splits each), 4 shares of 2644 rows 28 us. The partial sums are read as
+// waves are merged by the log-sum-exp rule, in a fixed order, the waves in pairs
+// (in one chain over 16 waves a context over 2000 positions was 2.00e-7 off 64
+// bits, now 1.88e-7; the same time). A prefill chunk has rows enough for one wave
+// each; a decode row (8 heads) takes as many waves as give each about four
+// partials. At 8192 positions 6.5 us (13.4 with 16 lanes per 4 dims walking 16 of
+// 256 splits each), 4 shares of 2644 rows 28 us. The partial sums are read as
 // 8-byte pairs (a partial is d + 2 floats).
 template <int W>
 __global__ __launch_bounds__(W < 4 ? 256 : 64 * W) void attention_combine_kernel(ReadArgs a) {
@@ -342,9 +344,10 @@ __global__ __launch_bounds__(W < 4 ? 256 : 64 * W) void attention_combine_kernel
     const int i = 4 * dl;
     const float* parts = a.parts + size_t(rh < total ? rh : 0) * a.splits * (a.d + 2);
     float m = -INFINITY, den = 0.f, num[4] = {0.f, 0.f, 0.f, 0.f};
+    // the factor that takes a sum from maximum `from` to `to` (-inf: nothing summed yet)
+    auto factor = [](float from, float to) { return from == -INFINITY ? 0.f : expf(from - to); };
     auto merge = [&](float mo, float dn, const float (&n)[4]) {
-        const float mn = fmaxf(m, mo);
-        const float c0 = m == -INFINITY ? 0.f : expf(m - mn), c1 = mo == -INFINITY ? 0.f : expf(mo - mn);
+        const float mn = fmaxf(m, mo), c0 = factor(m, mn), c1 = factor(mo, mn);
         den = den * c0 + dn * c1;
 #pragma unroll
         for (int e = 0; e < 4; ++e) num[e] = num[e] * c0 + n[e] * c1;
@@ -382,14 +385,23 @@ __global__ __launch_bounds__(W < 4 ? 256 : 64 * W) void attention_combine_kernel
         if (w != 0 || sl != 0) return;
 #pragma unroll
         for (int v = 1; v < W; ++v) m = fmaxf(m, sm[wb + v]);
-        den = num[0] = num[1] = num[2] = num[3] = 0.f;
+        float t[5][W];  // den and the four dims of every wave, added in pairs
 #pragma unroll
         for (int v = 0; v < W; ++v) {
-            const float c = sm[wb + v] == -INFINITY ? 0.f : expf(sm[wb + v] - m);
-            den += sd[wb + v] * c;
+            const float c = factor(sm[wb + v], m);
+            t[0][v] = sd[wb + v] * c;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) num[e] += sn[wb + v][e][dl] * c;
+            for (int e = 0; e < 4; ++e) t[1 + e][v] = sn[wb + v][e][dl] * c;
         }
+#pragma unroll
+        for (int n = W / 2; n > 0; n /= 2)
+#pragma unroll
+            for (int v = 0; v < n; ++v)
+#pragma unroll
+                for (int e = 0; e < 5; ++e) t[e][v] += t[e][v + n];
+        den = t[0][0];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) num[e] = t[1 + e][0];
     } else if (sl != 0) {
         return;
     }

@@ -132,3 +132,24 @@ def test_rows_of_eight_heads(both, length, rows):
     data = [rnd(rng, rows * heads * d), rnd(rng, n * kv * d), rnd(rng, n * kv * d), rnd(rng, rows * heads * d)]
     got, want = (read(b, d, heads, kv, length, rows, data) for b in both)
     parity(got, want, where=f"eight heads {length} {rows}")
+
+
+@pytest.mark.parametrize("length", [2000, 4000])
+def test_merge_adds_in_pairs(both, length):
+    """Equal scores over 125 splits of values in (0, 1): 16 waves' sums of even
+    size. Added in one chain they are off by 2.4e-8 sqrt(16 / 3) = 5.5e-8 (2.4e-8:
+    one rounding, 2-norm), in pairs by 2.4e-8 sqrt(1 + 1/2 + 1/4 + 1/8) = 3.3e-8;
+    the sums before and the division add 3e-8 (root of squares)."""
+    d, heads, kv = 256, 8, 2
+    rng = np.random.default_rng(length)
+    err = []
+    for _ in range(4):
+        values = rng.random((length, kv, d)).astype(np.float32)
+        data = [np.zeros(heads * d, np.float32), rnd(rng, length * kv * d), values.reshape(-1),
+                np.full(heads * d, 40.0, np.float32)]  # sigmoid(40) rounds to 1
+        got = read(both[0], d, heads, kv, length, 1, data).reshape(kv, heads // kv, d).astype(np.float64)
+        want = np.broadcast_to(values.astype(np.float64).mean(0)[:, None], got.shape)
+        err.append(np.sum((got - want) ** 2) / np.sum(want ** 2))
+    err = np.sqrt(np.mean(err))
+    print(f"error {err:.3e}", flush=True)
+    assert err < 5.3e-8
