@@ -810,17 +810,36 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     constexpr int P[6] = {2, 1, 0, 1, 0, 0}, Q[6] = {0, 1, 2, 0, 1, 0};  // part products, smallest first
     // this wave's partial scores of the tile in ks (its half of the dims)
     auto scores = [&](f16v& sc) {
+        // The leading products after all others: while the sum is small its roundings are too, and 8
+        // of 48 are left at its full size (2644 rows: 2.87e-7 off 64 bits with each step's six products
+        // together, now 2.21e-7; the time within 2 %). In a sum of their own, which the registers allow
+        // as well, the same error at 3 % more time: 16 additions more per tile beside the softmax.
+        auto key = [&](int p, int s) {
+            return *reinterpret_cast<const bf16x8*>(&ks[(p * 32 + lc) * B3_KROW + d0 + 16 * s + 8 * hl]);
+        };
 #pragma unroll
         for (int r = 0; r < 16; ++r) sc[r] = 0.f;
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
-            bf16x8 ka[3];
-#pragma unroll
-            for (int p = 0; p < 3; ++p)
-                ka[p] = *reinterpret_cast<const bf16x8*>(&ks[(p * 32 + lc) * B3_KROW + d0 + 16 * s + 8 * hl]);
-#pragma unroll
-            for (int pq = 0; pq < 6; ++pq) sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[P[pq]], qb[Q[pq]][s], sc, 0, 0, 0);
+            const bf16x8 k1 = key(1, s), k2 = key(2, s);
+            sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k2, qb[0][s], sc, 0, 0, 0);
+            sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k1, qb[1][s], sc, 0, 0, 0);
+            sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k1, qb[0][s], sc, 0, 0, 0);
         }
+        bf16x8 held[4];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {  // steps 4 .. 7, then 0 .. 3, whose plane 0 stays
+            const int s = (i + 4) & 7;
+            const bf16x8 k0 = key(0, s);
+            sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k0, qb[2][s], sc, 0, 0, 0);
+            sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k0, qb[1][s], sc, 0, 0, 0);
+            if (s < 4) held[s] = k0;
+        }
+        int again = 0;  // plane 0, its number hidden: steps 4 .. 7 are read again (kept: 16 registers more)
+        asm volatile("" : "+v"(again));
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+            sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(s < 4 ? held[s & 3] : key(again, s), qb[0][s], sc, 0, 0, 0);
     };
     // partial + the partner's (exchanged in xch) = the tile's scaled scores,
     // -inf at positions this lane's query does not see
@@ -1031,7 +1050,11 @@ bool bf3_shape(int d, int heads, int kv) { return d == 256 && kv > 0 && heads ==
 // 512 blocks (2644 rows: 4 shares 34.5 tiles, 3 shares 31; 128 rows over 2048
 // positions: 16 shares). Up to 2048 blocks, which bounds the partials. Measured
 // with the order of the blocks, 2644 tokens: this kernel 253 -> 201 us, the merge
-// 28 -> 26, an fp32 attention layer 519 -> 469 us (548 -> 496 on a slower card); 128 tokens over 1920 as before (its share count is the same).
+// 28 -> 26, an fp32 attention layer 519 -> 472 us (547 -> 498 on a slower card).
+// Fewer shares also mean longer sums in each; with the order of the products in
+// the kernel's scores no size measured is more than 2 % further off 64 bits than
+// with about 512 blocks and a step's products together (700 rows over 2644
+// cached, 5 shares instead of 8: 4.15e-7 and 4.14e-7).
 int bf3_splits(int rows, int heads, int kv, int tiles) {
     constexpr int kCus = 256;
     const int qt = ceil_div(rows, 32), first = tiles - qt > 0 ? tiles - qt : 0;  // tiles every row sees

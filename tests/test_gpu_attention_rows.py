@@ -153,3 +153,30 @@ def test_merge_adds_in_pairs(both, length):
     err = np.sqrt(np.mean(err))
     print(f"error {err:.3e}", flush=True)
     assert err < 5.3e-8
+
+
+@pytest.mark.parametrize("length,rows,bound", [(1, 128, 1.5e-7), (2001, 1000, 3.6e-7)])
+def test_prefill_read_error(both, length, rows, bound):
+    """The error of a chunk's read (2-norm, against float64). A score over 256
+    dims is two sums of 48 MFMAs; one rounding is about 2.4e-8 of the sum (2-norm)
+    and a sum grows as a random walk, so 48 at its size make 2.4e-8 sqrt(48 / 2) =
+    1.2e-7 of a score, the 8 leading products alone, after the others, 5e-8.
+    Measured here 1.95e-7 and 3.93e-7 with a step's six products together, 1.19e-7
+    and 3.19e-7 so; the contexts' own sums are the rest."""
+    d, heads, kv = 256, 8, 2
+    rng = np.random.default_rng(rows)
+    n = length + rows - 1
+    data = [rnd(rng, rows * heads * d), rnd(rng, n * kv * d), rnd(rng, n * kv * d), rnd(rng, rows * heads * d)]
+    got = read(both[0], d, heads, kv, length, rows, data).reshape(rows, heads, d)
+    q, k, v, gate = (x.astype(np.float64) for x in data)
+    q, k, v, gate = q.reshape(rows, heads, d), k.reshape(n, kv, d), v.reshape(n, kv, d), gate.reshape(rows, heads, d)
+    seen = np.arange(n)[None] < length + np.arange(rows)[:, None]
+    e2 = w2 = 0.0
+    for h in range(heads):
+        s = np.where(seen, q[:, h] @ k[:, h // 4].T / np.sqrt(d), -np.inf)
+        s = np.exp(s - s.max(1, keepdims=True))
+        want = (s / s.sum(1, keepdims=True)) @ v[:, h // 4] / (1 + np.exp(-gate[:, h]))
+        e2 += np.sum((got[:, h] - want) ** 2)
+        w2 += np.sum(want ** 2)
+    print(f"error {np.sqrt(e2 / w2):.3e}", flush=True)
+    assert np.sqrt(e2 / w2) < bound
