@@ -160,9 +160,9 @@ int qr_gemm_f32_add_norm(Context* c, float* y, const float* a, const float* x, i
  * tokens) runs gate, up and the silu product as one kernel, gate_y and up_y
  * untouched). Other column counts prepare nothing (returns 0). The planes are
  * dropped by qr_gemm_f32_release(a), by qr_free(a), and by any qr_write /
- * qr_copy into the matrix's range; unprepared matrices of up to a few
- * hundred tokens take gemm_kw.hip too (split or widened as they load), others
- * the split-BF16 kernel. */
+ * qr_copy into the matrix's range. Unprepared matrices over 5 to a few
+ * hundred tokens take gemm_kw.hip too (split or widened as they load; at most
+ * 16 rows: whole fp32 products), others the split-BF16 kernel. */
 int qr_gemm_f32_prepare(Context* c, const float* a, int rows, int cols);
 int qr_gemm_f32_release(Context* c, const float* a);
 /* Prepared BF16 matrices (no counterpart in the reference's ABI; optional,

@@ -9,8 +9,9 @@
 // (rows) output tile per 256-thread block, 2 x 2 waves of 64 x 64 (2 x 2 MFMA
 // tiles each); K in steps of 32 through LDS; the next K step's global loads are
 // in flight (registers) while the current one is multiplied.
-// fp32 weights with at most 16 rows (the DeltaNet a / b projections):
-// two such matrices per launch (x read once), up to 1024 columns, on fp32
+// fp32 weights with at most 16 rows (the DeltaNet a / b projections; up to 640
+// tokens only where no wider matrix of their group takes them along into
+// gemm_kw.hip): two such matrices per launch (x read once), up to 1024 columns, on fp32
 // MFMA (gemm_ab_mfma_kernel) for cols % 16 == 0, else gemm_ab_kernel; wider
 // rows: gemm_skinny_kernel (lanes over columns). BF16 and int8 weights of
 // that shape (cols % 16 == 0) take gemm_ab_mfma_kernel too.

@@ -21,8 +21,8 @@
 // tile a 64 x 64 tile moves 12 KiB for 24 MFMAs of fp32 weights (192 clocks
 // either way), a 32 x 32 tile 6 KiB for 6 MFMAs; weights read from HBM or
 // resident in the caches, in any k order, take the same time. A block's time
-// hardly depends on how many run beside it, so the tile is the smallest that
-// gives at most one block per CU (pick_tile).
+// hardly depends on how many run beside it, so the tile is the smallest of at
+// most 256 blocks (pick_tile); of a launch of more, two blocks run on a CU.
 //
 // Measured (one call, weights cold, launch included; before: the prefill GEMM
 // of gemm_p3.hip over planes, or gemm_bf3_kernel under 64 tokens and for
