@@ -151,12 +151,13 @@ struct Products<WeightType::F32> {
 };
 
 // n steps through a ring of NS (even) register buffers. step(buffer, step % 2,
-// next) multiplies a buffer and, for next >= 0, loads step `next` into it plane by plane as the products are done with it: loads issued in a burst after the
+// next) multiplies a buffer and, for next >= 0, loads step `next` into it plane
+// by plane as the products are done with it: loads issued in a burst after the
 // products stall the wave (the CU's vector memory path takes 16 clocks per KiB
 // and a wave issues in order), among them they do not: q|k|v of 128 fp32 tokens
-// 14.5 -> 12.0 us, of 300 25.8 -> 20.7, the BF16 GLU of 128 tokens 11.4 -> 10.3. The main loop's
-// loads are unconditional (a join between a path with loads and one without
-// would make the compiler wait for more than the buffer it needs).
+// 14.5 -> 12.0 us, of 300 25.8 -> 20.7, the BF16 GLU of 128 tokens 11.4 -> 10.3.
+// The main loop's loads are unconditional (a join between a path with loads and
+// one without would make the compiler wait for more than the buffer it needs).
 template <int NS, class Buf, class L, class S>
 __device__ __forceinline__ void ring(int n, L&& load, S&& step) {
     Buf b[NS];
@@ -617,7 +618,8 @@ int kw_gemm(hipStream_t s, WeightType t, const KwItem* items, int n, const __bf1
     if (M < 1 || n < 1 || n > kKwItems || !p3_cols_ok(K) || reinterpret_cast<uintptr_t>(x) % 16)
         return int(hipErrorInvalidValue);
     for (int i = 0; i < n; ++i)
-        if (items[i].rows < 1 || reinterpret_cast<uintptr_t>(items[i].scale) % 16 || !(kw_few_rows(items[i]) ? x != nullptr : xp != nullptr))
+        if (items[i].rows < 1 || reinterpret_cast<uintptr_t>(items[i].scale) % 16 ||
+            (kw_few_rows(items[i]) ? x == nullptr : xp == nullptr))
             return int(hipErrorInvalidValue);
     const Tile tile = pick_tile(t, items, n, M);
     KwArgs a{};
